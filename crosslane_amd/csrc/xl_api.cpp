@@ -1581,6 +1581,13 @@ void enqueue_shared(xl_context* ctx, int32_t type_gate, const void* d_gate, int3
     float* hd = reinterpret_cast<float*>(base + w.hd);
     const xl::MatRef mg = per32_matrix(type_gate, d_gate, ff, dim), mu = per32_matrix(type_up, d_up, ff, dim);
     const xl::MatRef md = per32_matrix(type_down, d_down, dim, ff);
+    // several tokens over dense matrices: the MFMA kernels, with the same bits
+    const hipError_t e = xl::dev::launch_ffn_tokens(mg, mu, md, T, dim, ff, d_x, d_out, xq, xd, hq, hd,
+                                                    ctx->cfg.swiglu_limit, ctx->err_flag, ctx->cus, s);
+    if (e != hipErrorNotSupported) {
+        hip_check(e, "shared FFN launch");
+        return;
+    }
     hip_check(xl::dev::launch_quant32(d_x, T, dim, xq, xd, ctx->err_flag, s), "quant32(x) launch");
     hip_check(xl::dev::launch_mv32(nullptr, nullptr, mg, mu, T, 0, 0, 2, ff, dim, xq, size_t(dim), xd,
                                    size_t(dim / 32), g, u, size_t(ff), ctx->tables, ctx->err_flag, s),

@@ -254,6 +254,16 @@ hipError_t launch_hc_post(const float* y, const float* res, const float* post, c
 // quantized per 32 into q, d exactly as launch_quant32 would quantize h.
 hipError_t launch_swiglu_quant32(const float* g, const float* u, int rows, int k, float lim, int8_t* q, float* d,
                                  hipStream_t s);
+// Shared-expert FFN of T tokens over dense matrices (xl_shared.hip), with the
+// bits of quant32, mv32, swiglu_quant32 and mv32 run token by token; xq, hq: T x
+// dim and T x ff bytes, xd, hd: a float per 32 of them. hipErrorNotSupported
+// below kFfnTokensMin tokens or for another block type.
+// Two tokens are still faster by the row kernels (29.5 against 34.8 us at 4096 x
+// 3072 of Q5_K / Q6_K; three: 36.6 against 35.3).
+constexpr int kFfnTokensMin = 3;
+hipError_t launch_ffn_tokens(const MatRef& gate, const MatRef& up, const MatRef& down, int T, int dim, int ff,
+                             const float* x, float* out, int8_t* xq, float* xd, int8_t* hq, float* hd, float lim,
+                             int* err, int cus, hipStream_t s);
 // h = SwiGLU(g, u) elementwise over n values, with the limit (lim <= 0: none).
 hipError_t launch_swiglu(const float* g, const float* u, int n, float lim, float* h, hipStream_t s);
 // Seeded generation of one planar matrix (role 0 gate, 1 up, 2 down).
