@@ -181,9 +181,9 @@ struct xl_context {
     struct Group {
         int32_t* ids = nullptr; float* w = nullptr; float* x = nullptr; float* shared = nullptr; float* out = nullptr;
         int8_t* xq = nullptr; float* xd = nullptr;
-        int32_t* order = nullptr; int32_t* pos = nullptr; int4* tasks = nullptr; int32_t* n_tasks = nullptr;
+        int32_t* order = nullptr; int32_t* pos = nullptr; int4* tasks = nullptr; int4* dtasks = nullptr;
+        xl::GroupQueue* queue = nullptr;
         float* h = nullptr; int8_t* hq = nullptr; float* hd = nullptr; float* y = nullptr;
-        uint64_t hq_bytes = 0;
     } grp;
     uint64_t* htag = nullptr;   // single-launch handoff buffers (Layer3Args)
     uint64_t* hqtag = nullptr;
@@ -670,23 +670,23 @@ int32_t xl_open(uint32_t abi_version, const xl_config* cfg, xl_context** out, xl
         if (cfg->max_tokens > 0) {
             const uint64_t T = uint64_t(cfg->max_tokens), GP = T * uint64_t(P);
             auto& g = ctx->grp;
-            const uint64_t slots = 16 * uint64_t(xl::group_max_tasks(int64_t(GP), cfg->n_experts));
-            g.hq_bytes = slots * uint64_t(ff);
+            const uint64_t tiles = uint64_t(xl::group_max_tiles(int64_t(GP), cfg->n_experts)), slots = 16 * tiles;
             const std::vector<Part> gparts = {
                 {reinterpret_cast<void**>(&g.ids), GP * 4},
                 {reinterpret_cast<void**>(&g.w), GP * 4},
                 {reinterpret_cast<void**>(&g.x), T * dim * 4},
                 {reinterpret_cast<void**>(&g.shared), T * dim * 4},
                 {reinterpret_cast<void**>(&g.out), T * dim * 4},
-                {reinterpret_cast<void**>(&g.xq), slots * dim},
-                {reinterpret_cast<void**>(&g.xd), T * (dim / 256) * 4},
+                {reinterpret_cast<void**>(&g.xq), slots * dim * 5 / 4},
+                {reinterpret_cast<void**>(&g.xd), slots * (dim / 256) * 4},
                 {reinterpret_cast<void**>(&g.order), slots * 4},
                 {reinterpret_cast<void**>(&g.pos), GP * 4},
-                {reinterpret_cast<void**>(&g.tasks), uint64_t(xl::group_max_tasks(int64_t(GP), cfg->n_experts)) * 16},
-                {reinterpret_cast<void**>(&g.n_tasks), 256},
+                {reinterpret_cast<void**>(&g.tasks), tiles * 16},
+                {reinterpret_cast<void**>(&g.dtasks), tiles * 16},
+                {reinterpret_cast<void**>(&g.queue), sizeof(xl::GroupQueue)},
                 {reinterpret_cast<void**>(&g.h), GP * ff * 4},
-                {reinterpret_cast<void**>(&g.hq), g.hq_bytes},
-                {reinterpret_cast<void**>(&g.hd), GP * (ff / 256) * 4},
+                {reinterpret_cast<void**>(&g.hq), slots * ff * 5 / 4},
+                {reinterpret_cast<void**>(&g.hd), slots * (ff / 256) * 4},
                 {reinterpret_cast<void**>(&g.y), GP * dim * 4},
             };
             parts.insert(parts.end(), gparts.begin(), gparts.end());
@@ -1118,18 +1118,22 @@ void enqueue_grouped(xl_context* ctx, int32_t layer, int32_t T, int32_t k, const
     const int gu_mask = ctx->gu_mask[size_t(layer)], dn_mask = ctx->dn_mask[size_t(layer)];
     Marks mark(ctx, s);
     mark("");
-    if (ctx->gpath != 0 && gu_mask == 1 && dn_mask == 2) {
+    // IQ2_XXS gate/up with IQ2_XS down always; layers of other types from kGroupAnyTokens
+    // tokens on (XL_GROUPED_PATH=2 and the trace are for the former only)
+    const bool iq2 = gu_mask == 1 && dn_mask == 2;
+    if (ctx->gpath != 0 && (iq2 || (ctx->gpath == 1 && !tr && T >= xl::kGroupAnyTokens))) {
         xl::GroupArgs a{};
         a.descs = ctx->d_descs + size_t(layer) * E;
         a.ids = d_ids; a.w = d_w; a.x = d_x; a.shared = d_shared; a.out = d_out;
         a.T = T; a.k = k; a.n_experts = E; a.dim = dim; a.ff = ctx->cfg.ff;
         const auto& g = ctx->grp;
-        a.xq = g.xq; a.xd = g.xd; a.order = g.order; a.pos = g.pos; a.tasks = g.tasks; a.n_tasks = g.n_tasks;
+        a.xq = g.xq; a.xd = g.xd; a.order = g.order; a.pos = g.pos; a.tasks = g.tasks; a.dtasks = g.dtasks;
+        a.queue = g.queue; a.cap = 16;
         a.h = g.h; a.hq = g.hq; a.hd = g.hd; a.y = g.y;
         a.tables = ctx->tables; a.err = ctx->err_flag;
         a.lim = ctx->cfg.swiglu_limit;
         if (tr) { a.tq8x = tr->q8x; a.tq8h = tr->q8h; a.tint = tr->ints; }
-        const hipError_t e = xl::dev::launch_grouped(a, ctx->cus, s);
+        const hipError_t e = xl::dev::launch_grouped(a, gu_mask, dn_mask, ctx->cus, s);
         if (e == hipSuccess) {
             if (tr && tr->h)   // the pairs' h as the gate/up kernel wrote it for Q8_K(h)
                 hip_check(hipMemcpyAsync(tr->h, g.h, sizeof(float) * size_t(T) * k * ctx->cfg.ff,

@@ -10,8 +10,7 @@
 //                    at most 16 pairs of one expert
 //   q8k_rows_kernel  Q8_K (q8k_core.hpp:30-38) of token rows (x) and pair rows
 //                    (h), written in the operand order of the MFMA kernels
-//   gu_kernel        gate/up + SwiGLU of every task (IQ2_XXS)
-//   dn_kernel        down of every task (IQ2_XS)
+//   grouped_kernel   gate/up + SwiGLU of every task, then down of every task
 //   gcombine_kernel  fixed-order combine per token, + shared
 //
 // MFMA: v_mfma_i32_16x16x32_i8 with M = pairs, N = weight rows, K = the 32
@@ -23,15 +22,41 @@
 // partials are exact. Any K order works as long as A and B agree, which the
 // chunk-major activation layouts below guarantee.
 //
-// Weights stream from HBM through registers: each wave loads its 16 rows' next
-// block while it computes the current one, and touches the line four blocks
-// ahead with one dword per row so that it is in L2 when the real loads come.
-// The texture data path costs one cycle per cache access, and a quad of lanes
-// makes one access only when it reads 64 contiguous bytes: so each lane loads
-// just the 16 B of its row's block that it decodes (the entries then move
-// between lane groups by permlane swaps), activations are laid out so that a
-// quad's four slots are adjacent, and the small per-block scales are staged in
-// LDS once per work item instead of being loaded by every wave.
+// IQ1_M needs neither: its sub-scale (2s + 1 <= 15) times its grid value (-1, 0, 1)
+// is an int8 (the LDS table holds byte selectors, v_perm picks the scale, its
+// negative or zero by them), so that a block's eight MFMAs accumulate into one
+// result, and any lane may hold any of the block's entries (lane group e4 keeps
+// values 64 e4 .. + 63: the activations have an order of their own). The delta term, (2s + 1) * (+-1) times
+// the sum of an entry's 8 quants, is a product over the block's 32 entries: two
+// more MFMAs on those sums (11 bits, split 16 hi + lo by the quantizer).
+//
+// Work: a wave takes one tile at a time, two streams of 16 rows that share the
+// activations (gate and up rows, or 32 down rows), from its workgroup's current
+// bundle; a wave that finds the bundle empty fetches the next one from the
+// device's queue of the type. Waves never wait for each other inside a type (a
+// workgroup barrier per item left every wave waiting for the item's chain of
+// dependent loads: task, matrix, scales, weights). A layer of several types has
+// one queue per type; a workgroup starts with the type its place in the grid falls
+// on (by estimated cost) and goes on with the others' remainders, each after
+// filling its LDS tables for that type.
+//
+// Weights stream from HBM through registers: each wave loads its rows' next block
+// while it computes the current one, and touches the line four blocks ahead with
+// one dword per row so that it is in L2 when the real loads come. The texture data
+// path costs one cycle per cache access, and a quad of lanes makes one access only
+// when it reads 64 contiguous bytes: so each lane loads just the 16 B of its row's
+// block that it decodes (the entries then move between lane groups by permlane
+// swaps), activations are laid out so that a quad's four slots are adjacent, and
+// the small per-block scales are staged once per tile in the wave's own LDS. An
+// IQ1_M lane needs 8, 4 and 8 bytes of three planes per block: loaded directly,
+// those kept the texture unit busy for the whole kernel (1,415 us for gate/up of
+// 512 tokens at 4096 x 3072, 384 experts), so four blocks of the 16 rows come as
+// whole 16-byte pieces and go through the wave's LDS.
+//
+// Bound by the decode work per weight byte: at 512 tokens (4096 x 3072, 384 experts,
+// 6 picks) the IQ2 gate/up launch issues VALU on 71 % of its cycles, LDS lookups fill
+// 38 %. Whole calls there: IQ2 1,422 us (1,463 with workgroup barriers per item),
+// IQ1_M 1,265, mixed types 1,426 (10,999 and 12,992 as 512 layer calls).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -45,32 +70,39 @@ namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-constexpr int kTile = 16;   // pairs per task (the MFMA M dimension)
+constexpr int kTile = 16;   // pairs per tile (the MFMA M dimension)
+// GroupArgs::pos: slot of a pair, and whether its x / h go there in the IQ1_M order.
+constexpr int kSlotX1 = 1 << 30, kSlotH1 = 1 << 29, kSlotMask = kSlotH1 - 1;
+// Relative cost of a tile by type (XXS, XS, IQ1_M), for the first share of a mixed
+// layer's workgroups (the queues even out what it misses).
+__device__ constexpr int kTileCost[3] = {10, 11, 8};
 // Expanded codebook tables (layer_tables() in xl_api.cpp): 128 sign entries of
 // 16 B (byte mask, then the mask's low bits), the IQ2_XXS grid (256 x 8 B), the
 // IQ2_XS grid (512 x 8 B).
 constexpr int kTabSgn = 0, kTabXXS = 2048, kTabXS = 4096;
 
-// LDS of the MFMA kernels: grid entries as 16 B (g, -g) in C copies per entry
-// (lane copy = lane % C, so the 16 lanes of one ds_read_b128 pass never share
-// a bank), sign masks as 8 B in 32 copies (the 32 lanes of one ds_read_b64 pass
-// never share a bank) indexed by a whole byte whose top bit is not a sign bit.
-constexpr int kL_GRID = 0, kL_SGN = 65536, kL_TAB = 131072;
-// Per work item, staged once by the workgroup (each wave would otherwise issue
-// these small loads every block): the 16 pairs' activation block scales
-// [block][pair] (f32), then the item's rows' fp16 block scales [row][block]
-// for each matrix (NW x 16 rows), then (down) the rows' IQ2_XS scale bytes
-// [row][block][8].
-// Blocks per row these regions hold: gate/up rows of dim <= kMaxRowK, down
-// rows of ff <= 4096.
-constexpr int kGuNb = kMaxRowK / 256, kDnNb = 16;
-constexpr int kL_PD = kL_TAB;
-constexpr int kL_RDG = kL_PD + 16 * kGuNb * 4;     // gate/up: 2 planes of `rows` rows x kGuNb fp16 scales
-constexpr int gu_lds_bytes(int rows) { return kL_RDG + 2 * rows * kGuNb * 2; }
-constexpr int kL_RDD = kL_PD + 16 * kDnNb * 4;     // down: `rows` rows x kDnNb fp16 scales, then scale bytes
-constexpr int dn_rs(int rows) { return kL_RDD + rows * kDnNb * 2; }
-constexpr int dn_lds_bytes(int rows) { return dn_rs(rows) + rows * kDnNb * 8; }
-static_assert(gu_lds_bytes(12 * 16) <= 160 * 1024 && dn_lds_bytes(12 * 16) <= 160 * 1024, "LDS budget");
+// LDS tables of one type (128 KB). IQ2: grid entries as 16 B (g, -g) in C copies
+// per entry (lane copy = lane % C, so the 16 lanes of one ds_read_b128 pass never
+// share a bank), then sign masks as 8 B in 32 copies (the 32 lanes of one
+// ds_read_b64 pass never share a bank) indexed by a whole byte whose top bit is not
+// a sign bit. IQ1_M (16 KB): the grid as 8 B of v_perm selectors (0: 1, 1: -1, 0x0C: 0).
+constexpr int kL_GRID = 0, kL_SGN = 65536, kL_TAB = 131072, kL_TAB1 = 16384;
+constexpr int kTabIQ1 = 8192;   // IQ1 grid in the expanded tables
+// Then each wave's staging: its tile's 16 pairs' activation scales [block][tile
+// position] (f32), then its two streams' fp16 row scales [row][block].
+constexpr int kGrpNb = kMaxRowK / 256;
+constexpr int kL_WAVE = 64 * kGrpNb + 2 * 16 * kGrpNb * 2;
+// IQ1_M waves: the activation scales, then per stream four blocks of 16 rows:
+// [block][row] 32 B of indices, then 16 B of nibbles, then 8 B of scale words.
+// (block strides a quarter more than the 512, 256 and 128 bytes: the pieces of one
+// store then fall into different banks)
+constexpr int kR1q = 576, kR1h = 320, kR1s = 192, kR1ho = 4 * kR1q, kR1so = kR1ho + 4 * kR1h;
+constexpr int kRaw1 = kR1so + 4 * kR1s, kL_WAVE1 = 64 * kGrpNb + 2 * kRaw1;
+constexpr int grp_lds_bytes(int mask, int nw) {
+    const int iq2 = mask & 3 ? kL_TAB + nw * kL_WAVE : 0, iq1 = mask & 4 ? kL_TAB1 + nw * kL_WAVE1 : 0;
+    return iq2 > iq1 ? iq2 : iq1;
+}
+static_assert(grp_lds_bytes(7, 12) + 64 <= 160 * 1024, "LDS budget");
 constexpr int kCopiesXXS = 16;   // 256 entries x 256 B: the entry byte lands in address byte 1
 constexpr int kCopiesXS = 8;     // 512 entries x 128 B: the 9-bit entry lands at address bit 7
 
@@ -132,18 +164,63 @@ __device__ __forceinline__ void fill_grid(uint8_t* lds, const uint64_t* grid, in
     }
 }
 
+// The tables of block type ty.
+template <int NT>
+__device__ __forceinline__ void fill_tables(uint8_t* lds, int ty, const uint64_t* tab, int t) {
+    if (ty == kIQ2_XXS) {
+        fill_grid<256, kCopiesXXS>(lds, tab + kTabXXS / 8, t, NT);
+        fill_signs(lds, tab, t, NT);
+    } else if (ty == kIQ2_XS) {
+        fill_grid<512, kCopiesXS>(lds, tab + kTabXS / 8, t, NT);
+        fill_signs(lds, tab, t, NT);
+    } else {
+        constexpr uint64_t kOnes = 0x0101010101010101ull;
+        for (int i = t; i < 2048; i += NT) {
+            const uint64_t g = tab[kTabIQ1 / 8 + i], n = (g >> 1) & kOnes;   // bytes 0xff
+            *reinterpret_cast<uint64_t*>(lds + 8 * i) = (kOnes ^ (g & kOnes)) * 0x0Cu + n;
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
-// Buckets: counts per expert in LDS, one scan of pairs and tasks, then each
-// valid pair takes a slot of its expert's tasks (task i: slots 16 i .. + 15).
-// The slot order inside an expert varies run to run; no result depends on it
-// (every output of a pair is computed from that pair's operands only, in a
-// fixed order).
+// Buckets: counts per expert in LDS, one scan of tiles and tasks, then each valid
+// pair takes a slot of its expert's tiles (tile i: slots 16 i .. + 15). A task is
+// up to a.cap pairs of one expert, in consecutive tiles. The tasks are listed
+// twice, by the expert's gate type and by its down type (kIQ2_XXS, kIQ2_XS,
+// kIQ1_M in turn), each list's type counts beside it. The slot order inside an
+// expert varies run to run; no result depends on it (every output of a pair is
+// computed from that pair's operands only, in a fixed order).
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ int type_index(int t) { return t == kIQ2_XXS ? 0 : t == kIQ2_XS ? 1 : 2; }
+// One count per type in 21 bits each (tasks of a call are below 2^17).
+__device__ __forceinline__ uint64_t type_count(int ti, int n) { return uint64_t(uint32_t(n)) << (21 * ti); }
+__device__ __forceinline__ int type_part(uint64_t v, int ti) { return int((v >> (21 * ti)) & 0x1fffff); }
+// Inclusive scan over the workgroup's 1024 threads; sh: 17 words (the total last).
+__device__ __forceinline__ uint64_t scan1024(uint64_t v, uint64_t* sh, int t) {
+    const int lane = t & 63, wv = t >> 6;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint64_t u = __shfl_up(v, o);
+        if (lane >= o) v += u;
+    }
+    __syncthreads();   // an earlier scan's words are read
+    if (lane == 63) sh[wv] = v;
+    __syncthreads();
+    uint64_t before = 0;
+    for (int i = 0; i < wv; ++i) before += sh[i];
+    v += before;
+    if (t == 1023) sh[16] = v;
+    __syncthreads();
+    return v;
+}
 __global__ __launch_bounds__(1024) void bucket_kernel(GroupArgs a) {
     __shared__ int cnt[kGroupMaxExperts];
     __shared__ int cur[kGroupMaxExperts];
-    __shared__ int part[2 * 1024];
+    __shared__ uint64_t sh[17];
     const int t = threadIdx.x, P = a.T * a.k, E = a.n_experts;
+    // this thread's first expert's types, loaded under the counting
+    const int ef = min(E - 1, t * ((E + 1023) / 1024));
+    const int g_first = a.descs[ef].m[0].type, d_first = a.descs[ef].m[2].type;
     for (int e = t; e < E; e += 1024) cnt[e] = 0;
     __syncthreads();
     for (int p = t; p < P; p += 1024) {
@@ -152,33 +229,64 @@ __global__ __launch_bounds__(1024) void bucket_kernel(GroupArgs a) {
         else atomicOr(a.err, kDevErrExpertId);
     }
     __syncthreads();
+    const auto gate_type = [&](int e) { return type_index(e == ef ? g_first : a.descs[e].m[0].type); };
+    const auto down_type = [&](int e) { return type_index(e == ef ? d_first : a.descs[e].m[2].type); };
     const int per = (E + 1023) / 1024, e0 = min(E, t * per), e1 = min(E, e0 + per);
-    int st = 0;
-    for (int e = e0; e < e1; ++e) st += (cnt[e] + kTile - 1) / kTile;
-    part[t] = st;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {   // inclusive scan of tasks
-        const int v = t >= off ? part[t - off] : 0;
-        __syncthreads();
-        part[t] += v;
-        __syncthreads();
+    uint64_t tiles = 0, gu = 0, dn = 0;
+    for (int e = e0; e < e1; ++e) {
+        const int c = cnt[e], n = (c + a.cap - 1) / a.cap;
+        tiles += uint64_t((c + kTile - 1) / kTile) | (uint64_t(n) << 32);
+        gu += type_count(gate_type(e), n);
+        dn += type_count(down_type(e), n);
     }
-    int bt = part[t] - st;
+    const uint64_t tt = scan1024(tiles, sh, t) - tiles;   // tiles, tasks << 32
+    int tile = int(uint32_t(tt));
+    uint64_t g_at, g_all, d_at, d_all;
+    if (a.gu_first && a.dn_first) {   // one type each: their lists are the tasks in turn
+        const int gt = type_index(g_first), dt = type_index(d_first);
+        g_at = type_count(gt, int(tt >> 32));
+        d_at = type_count(dt, int(tt >> 32));
+        g_all = type_count(gt, int(sh[16] >> 32));
+        d_all = type_count(dt, int(sh[16] >> 32));
+    } else {
+        g_at = scan1024(gu, sh, t) - gu;
+        g_all = sh[16];
+        d_at = scan1024(dn, sh, t) - dn;
+        d_all = sh[16];
+    }
+    // the types' lists one after the other
+    const uint64_t g0 = type_count(1, type_part(g_all, 0)) + type_count(2, type_part(g_all, 0) + type_part(g_all, 1));
+    const uint64_t d0 = type_count(1, type_part(d_all, 0)) + type_count(2, type_part(d_all, 0) + type_part(d_all, 1));
+    g_at += g0;
+    d_at += d0;
     for (int e = e0; e < e1; ++e) {
         const int c = cnt[e];
-        for (int i = 0; i * kTile < c; ++i)
-            a.tasks[bt + i] = make_int4(e, kTile * (bt + i), min(kTile, c - kTile * i), 0);
-        cur[e] = kTile * bt;   // the expert's first slot; its pairs fill its tasks' slots in turn
-        bt += (c + kTile - 1) / kTile;
+        const int gt = gate_type(e), dt = down_type(e);
+        // the expert's first slot; its pairs fill its tiles' slots in turn. Bits 30
+        // and 29: x and h in the IQ1_M order
+        cur[e] = (kTile * tile) | (gt == 2 ? kSlotX1 : 0) | (dt == 2 ? kSlotH1 : 0);
+        for (int i = 0; i * a.cap < c; ++i) {
+            const int4 task = make_int4(e, kTile * tile, min(a.cap, c - a.cap * i), 0);
+            a.tasks[type_part(g_at, gt)] = task;
+            a.dtasks[type_part(d_at, dt)] = task;
+            g_at += type_count(gt, 1);
+            d_at += type_count(dt, 1);
+            tile += (task.z + kTile - 1) / kTile;
+        }
     }
-    if (t == 1023) *a.n_tasks = part[1023];
+    if (t < 3) {
+        a.queue->gu_tasks[t] = type_part(g_all, t);
+        a.queue->dn_tasks[t] = type_part(d_all, t);
+        a.queue->gu_next[t] = a.gu_first;
+        a.queue->dn_next[t] = a.dn_first;
+    }
     __syncthreads();
     for (int p = t; p < P; p += 1024) {
         const int e = a.ids[p];
         int slot = -1;
         if (e >= 0 && e < E) {
-            slot = atomicAdd(&cur[e], 1);   // consecutive per expert: its tasks' slots have no gaps before the last
-            a.order[slot] = p;
+            slot = atomicAdd(&cur[e], 1);   // consecutive per expert: its tiles' slots have no gaps before the last
+            a.order[slot & kSlotMask] = p;
         }
         a.pos[p] = slot;
     }
@@ -188,24 +296,26 @@ __global__ __launch_bounds__(1024) void bucket_kernel(GroupArgs a) {
 // Q8_K of 256-value blocks of rows, one wave per block, written to the slots of
 // the row's pairs (ROWS_X: a token row goes to its k pairs' slots; ROWS_H: a
 // pair row to its slot; bad ids have none) in the operand order of the MFMA
-// kernels. Task i's slots form one region of nb * 4 KiB; in it, per block b,
-// the 16-B piece i of chunk e (the 8 quants of entry e of sub-blocks 2i and
-// 2i + 1) of slot s sits at ((4 b + i) * 4 + e) * 256 + 16 s, so that four lanes
-// of consecutive slots read 64 contiguous bytes.
+// kernels. A tile's slots form one region of nb * 5 KiB; in its first nb * 4 KiB,
+// per block b, the 16-B piece i of chunk e of slot s sits at ((4 b + i) * 4 + e) *
+// 256 + 16 s, so that four lanes of consecutive slots read 64 contiguous bytes.
+// IQ2 order: piece i of chunk e is the 8 quants of entry e of sub-blocks 2i and
+// 2i + 1. IQ1_M order: chunk e is values 64 e .. + 63, piece i 16 of them; then, in
+// the region's last nb KiB, the sums S of each 8 values as S = 16 hi + lo: slot
+// s's 16 bytes at (4 b + e) * 256 + 16 s hold lo, then hi, of chunk e's entries 0, 2,
+// 4, 6, 1, 3, 5, 7. The block scale goes to the tile's [block][slot] floats.
 // ---------------------------------------------------------------------------
-// The j-th pair of a task (slot 16 i + j) sits at tile position 4 (j % 4) + j / 4
+// The j-th pair of a tile (slot 16 i + j) sits at tile position 4 (j % 4) + j / 4
 // (M index of the MFMAs; the map is its own inverse): the lane holding M rows
-// 4 e + r, r = 0..3, gets pairs 4 r + e, so a task of n pairs has results only
+// 4 e + r, r = 0..3, gets pairs 4 r + e, so a tile of n pairs has results only
 // in the lanes' first ceil(n / 4) output registers.
 __device__ __forceinline__ int tile_pos(int j) { return ((j & 3) << 2) | (j >> 2); }
-__device__ __forceinline__ size_t slot_off(int slot, int nb, int blk, int piece, int chunk) {
-    return size_t(slot >> 4) * size_t(nb) * 4096 +
-           size_t(((4 * blk + piece) * 4 + chunk) * 256 + 16 * tile_pos(slot & 15));
-}
+__device__ __forceinline__ size_t tile_off(int tile, int nb) { return size_t(tile) * size_t(nb) * 5120; }
 enum { ROWS_X = 0, ROWS_H = 1 };
 // trace (null outside the parity trace): the row's blocks also as 292-byte Q8_K
 // blocks, row-major (a token's for ROWS_X, a pair's for ROWS_H).
-template <int MODE, bool TR>
+// IQ1: some slots may be in the IQ1_M order.
+template <int MODE, bool IQ1, bool TR>
 __global__ __launch_bounds__(256) void q8k_rows_kernel(const float* __restrict__ src, int rows, int nb,
                                                        int8_t* __restrict__ q, float* __restrict__ d,
                                                        const int32_t* __restrict__ pos, int k,
@@ -219,13 +329,32 @@ __global__ __launch_bounds__(256) void q8k_rows_kernel(const float* __restrict__
     const float v[4] = {v4.x, v4.y, v4.z, v4.w};
     const Q8Lane r = q8k_lane(v, lane);
     if (!r.finite && lane == 0) atomicOr(err, kDevErrNonFinite);
-    const int c = lane >> 3, e = (lane >> 1) & 3, j = 8 * (c & 1) + 4 * (lane & 1);   // values 4 lane .. + 3
+    // values 4 lane .. + 3 in the IQ2 order: sub-block c, entry e
+    const int c = lane >> 3, e = (lane >> 1) & 3;
+    const int o2 = ((4 * blk + (c >> 1)) * 4 + e) * 256 + 8 * (c & 1) + 4 * (lane & 1);
+    // in the IQ1_M order: chunk lane / 16, piece (lane / 4) % 4; its entry's sum
+    const int o1 = ((4 * blk + ((lane >> 2) & 3)) * 4 + (lane >> 4)) * 256 + 4 * (lane & 3);
+    int sum = __builtin_amdgcn_sdot4(int(r.packed), 0x01010101, 0, false);
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0xB1, 0xF, 0xF, false);   // lane ^ 1: the entry's 8 values
+    const int j = (lane >> 1) & 7, lo = ((sum + 8) & 15) - 8, hi = (sum - lo) >> 4;
+    const int os = nb * 4096 + (4 * blk + (lane >> 4)) * 256 + (j >> 1) + 4 * (j & 1);
     const int np = MODE == ROWS_X ? k : 1;
     for (int i = 0; i < np; ++i) {
         const int slot = pos[MODE == ROWS_X ? row * k + i : row];
-        if (slot >= 0) *reinterpret_cast<uint32_t*>(q + slot_off(slot, nb, blk, c >> 1, e) + j) = r.packed;
+        if (slot < 0) continue;
+        const int s = slot & kSlotMask, tp = tile_pos(s & 15);
+        int8_t* t = q + tile_off(s >> 4, nb) + 16 * tp;
+        if (IQ1 && (slot & (MODE == ROWS_X ? kSlotX1 : kSlotH1))) {
+            *reinterpret_cast<uint32_t*>(t + o1) = r.packed;
+            if (!(lane & 1)) {
+                t[os] = int8_t(lo);
+                t[os + 8] = int8_t(hi);
+            }
+        } else {
+            *reinterpret_cast<uint32_t*>(t + o2) = r.packed;
+        }
+        if (lane == 0) d[(size_t(s >> 4) * nb + blk) * 16 + tp] = r.d;
     }
-    if (lane == 0) d[b] = r.d;
     if constexpr (TR) {
         if (trace) trace_q8_block(trace + size_t(b) * 292, r.d, r.packed, lane);
     }
@@ -255,11 +384,6 @@ __device__ __forceinline__ uint32_t ld32(__amdgpu_buffer_rsrc_t r, uint32_t v, u
 __device__ __forceinline__ uint16_t ld16(__amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t so = 0) {
     return __builtin_amdgcn_raw_buffer_load_b16(r, v, so, 0);
 }
-
-// One block's operands for one wave.
-struct GuOps {
-    uint4 g, u, a[4];   // 16-B part e4 of the row's gate / up block, the lane's activation chunk
-};
 
 // Exchanges across the four 16-lane groups (e4 = lane / 16) of a wave.
 __device__ __forceinline__ void swap32(uint32_t& x, uint32_t& y) {   // lanes 32.. of x <-> lanes ..31 of y
@@ -314,190 +438,6 @@ __device__ __forceinline__ XxsLane xxs_lane(const uint4& w, int e4) {
     r.ls[1] = ((s >> 3) & 0x1E1E1E1Eu) | 0x01010101u;
     return r;
 }
-struct DnOps {
-    uint4 q, a[4];      // 16-B part e4 of the row's down block, the lane's activation chunk
-};
-
-// Stages one item's pair scales (scl: one f32 per (pair row, block), pairs of
-// the task's order slots) and `mats` planes of fp16 row scales (rows rows from
-// row0, nb per row, contiguous in each plane) into LDS, after a barrier.
-// The planes go to LDS at rd, `mstride` bytes apart.
-template <int NT>
-__device__ __forceinline__ void stage_item(uint8_t* lds, const GroupArgs& a, const int4& tk, const float* scl, int per_pair,
-                                           int nb, const uint8_t* const* planes, int mats, int row0, int rows, int t,
-                                           int rd, int mstride) {
-    __syncthreads();   // every wave is done with the previous item's staging
-    for (int i = t; i < 16 * nb; i += NT) {
-        const int pos = i & 15, blk = i >> 4;   // tile position pos holds the task's pair tile_pos(pos)
-        const int p = a.order[tk.y + min(tile_pos(pos), tk.z - 1)];
-        reinterpret_cast<float*>(lds + kL_PD)[i] = scl[size_t(per_pair ? p : p / a.k) * nb + blk];
-    }
-    const int chunks = rows * nb * 2 / 16;   // 16-byte pieces of one plane's rows
-    for (int i = t; i < mats * chunks; i += NT) {
-        const int m = i / chunks, c = i - m * chunks;
-        const uint4 v = reinterpret_cast<const uint4*>(planes[m] + size_t(row0) * nb * 2)[c];
-        *reinterpret_cast<uint4*>(lds + rd + m * mstride + 16 * c) = v;
-    }
-}
-
-// ---------------------------------------------------------------------------
-// gate/up + SwiGLU. Work item = (task, group of NW * 16 rows); wave wv owns
-// rows 16 wv .. + 15 of the group in gate and up.
-// ---------------------------------------------------------------------------
-// TR: also write each pair's block integers (GroupArgs::tint).
-template <int NW, bool TR>
-__global__ __launch_bounds__(NW * 64, 1) void gu_kernel(GroupArgs a) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[gu_lds_bytes(NW * 16)];
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    fill_grid<256, kCopiesXXS>(lds, a.tables + kTabXXS / 8, t, NW * 64);
-    fill_signs(lds, a.tables, t, NW * 64);
-    __syncthreads();
-
-    const int col = lane & 15, e4 = lane >> 4;
-    const int nb = a.dim / 256, groups = a.ff / (NW * 16);
-    const int items = uni(*a.n_tasks) * groups;
-    const uint32_t lo_g = uint32_t(lane & (kCopiesXXS - 1)) << 4;        // kL_GRID = 0
-    const uint32_t lo_s = (uint32_t(lane & 31) << 3) | (1u << 16);       // kL_SGN = 1 << 16
-    uint32_t sunk = 0;
-    for (int item = blockIdx.x; item < items; item += gridDim.x) {
-        const int task = item / groups, grp = item - task * groups;
-        const int4 tk = task_at(a.tasks, task);
-        const int row = grp * NW * 16 + wv * 16 + col;
-        // A operand: slot col of the task (past its pairs: unused slot memory, whose
-        // outputs are discarded), the lane's chunk e4, block 0
-        const uint32_t va = uint32_t(slot_off(tk.y, nb, 0, 0, e4) + 16 * col);
-        int po[4];   // the pairs of the lane's four outputs (tile positions 4 e4 + r)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int j = 4 * r + e4;
-            po[r] = j < tk.z ? a.order[tk.y + j] : -1;
-        }
-        const MatRef G = mat_at(a.descs, tk.x, 0), U = mat_at(a.descs, tk.x, 1);
-        {
-            const uint8_t* planes[2] = {G.base + G.off1, U.base + U.off1};
-            stage_item<NW * 64>(lds, a, tk, a.xd, 0, nb, planes, 2, grp * NW * 16, NW * 16, t, kL_RDG,
-                                NW * 16 * kGuNb * 2);
-        }
-        const __amdgpu_buffer_rsrc_t rg = rsrc(G.base), ru = rsrc(U.base), rx = rsrc(a.xq);
-        const uint32_t vq = uint32_t(row * nb) * 64u;
-        auto load = [&](GuOps& o, int blk) {
-            o.g = ld128(rg, vq + 64u * blk + 16u * e4);
-            o.u = ld128(ru, vq + 64u * blk + 16u * e4);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o.a[i] = ld128(rx, va + 4096u * blk + 1024u * i);
-        };
-        auto touch = [&](int blk) { return ld32(rg, vq + 64u * blk) ^ ld32(ru, vq + 64u * blk); };
-        // RR: output registers that can hold a pair (2 for tasks of at most 8 pairs, else 4)
-        auto run = [&]<int RR>() {
-            float accg[4] = {0.0f, 0.0f, 0.0f, 0.0f}, accu[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            // Sub-block c of a matrix: its grid entry (g, -g) and sign mask from LDS,
-            // then B = signed entry, one MFMA, the row's (2s + 1) on the RR outputs.
-            // All eight gate lookups are issued first; each up lookup is issued as a
-            // gate one is consumed, so about seven are in flight throughout.
-            struct Look { uint4 g; uint2 m; };
-            auto look = [&](const XxsLane& X, int c) {   // grid byte -> address byte 1, then the aux byte
-                const uint32_t w = X.u[c >> 1], h = uint32_t(c & 1) * 2u;
-                Look L;
-                L.g = *reinterpret_cast<const uint4*>(lds + perm(w, lo_g, 0x0C020000u | ((4u + h) << 8)));
-                L.m = *reinterpret_cast<const uint2*>(lds + perm(w, lo_s, 0x0C020000u | ((5u + h) << 8)));
-                return L;
-            };
-            auto prod = [&](const Look& L, long A) {
-                return mfma(A, pack64(bfi(L.m.x, L.g.z, L.g.x), bfi(L.m.y, L.g.w, L.g.y)), v4i{0, 0, 0, 0});
-            };
-            auto scale = [&](const v4i& C, const XxsLane& X, int c, int (&bi)[4]) {
-                const int ls = int(__builtin_amdgcn_ubfe(X.ls[c & 1], 8 * (c >> 1), 8));
-#pragma unroll
-                for (int r = 0; r < RR; ++r) bi[r] = mad24(ls, C[r], bi[r]);
-            };
-            const uint16_t* sdg = reinterpret_cast<const uint16_t*>(lds + kL_RDG) + (wv * 16 + col) * nb;
-            const uint16_t* sdu = sdg + NW * 16 * kGuNb;
-            int blk_c = 0;   // block the next compute() handles
-            auto compute = [&](const GuOps& o) {
-                const int b = blk_c++;
-                int big[4] = {0, 0, 0, 0}, biu[4] = {0, 0, 0, 0};
-                long A[8];
-#pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    const uint32_t* av = reinterpret_cast<const uint32_t*>(o.a) + 2 * c;
-                    A[c] = pack64(av[0], av[1]);
-                }
-                const XxsLane XG = xxs_lane(o.g, e4), XU = xxs_lane(o.u, e4);
-                Look L[8];
-#pragma unroll
-                for (int c = 0; c < 8; ++c) L[c] = look(XG, c);
-                // step i < 8: gate sub-block i, else up sub-block i - 8; each step's
-                // MFMA is issued before the previous step's multiply-adds read theirs
-                v4i C[16];
-#pragma unroll
-                for (int i = 0; i <= 16; ++i) {
-                    if (i < 8) {
-                        C[i] = prod(L[i], A[i]);
-                        L[i] = look(XU, i);
-                    } else if (i < 16) {
-                        C[i] = prod(L[i - 8], A[i - 8]);
-                    }
-                    if (i > 8) scale(C[i - 1], XU, i - 9, biu);
-                    else if (i > 0) scale(C[i - 1], XG, i - 1, big);
-                }
-                if constexpr (TR) {   // pair po[r]'s block integers of this lane's row
-                    const size_t rec = 2 * size_t(a.ff) * nb + size_t(a.dim) * (a.ff / 256);
-#pragma unroll
-                    for (int r = 0; r < RR; ++r)
-                        if (a.tint && po[r] >= 0) {
-                            const size_t o = size_t(po[r]) * rec + size_t(row) * nb + size_t(b);
-                            a.tint[o] = big[r];
-                            a.tint[o + size_t(a.ff) * nb] = biu[r];
-                        }
-                }
-                const float dgf = h2f(sdg[b]), duf = h2f(sdu[b]);
-                const float4 xd4 = *reinterpret_cast<const float4*>(lds + kL_PD + 64 * b + 16 * e4);
-                const float xd[4] = {xd4.x, xd4.y, xd4.z, xd4.w};
-#pragma unroll
-                for (int r = 0; r < RR; ++r) {
-                    accg[r] = fmaf(__fmul_rn(dgf, xd[r]), float(big[r]), accg[r]);
-                    accu[r] = fmaf(__fmul_rn(duf, xd[r]), float(biu[r]), accu[r]);
-                }
-            };
-            // Two operand sets alternate over a 4-step unrolled loop (no register
-            // copies, so no wait ever covers a load issued in the same step); line
-            // touches four blocks ahead in four fixed registers.
-            // A row's blocks 2j and 2j + 1 share a 128-byte line: one touch per line.
-            GuOps s0, s1;
-            load(s0, 0);
-            uint32_t t0 = touch(min(1, nb - 1)), t2 = touch(min(3, nb - 1));
-            for (int b = 0; b < nb; b += 4) {
-                load(s1, min(b + 1, nb - 1));
-                sink(sunk, t0);
-                t0 = touch(min(b + 5, nb - 1));
-                __builtin_amdgcn_sched_barrier(0);   // the loads stay ahead of the compute
-                compute(s0);
-                load(s0, min(b + 2, nb - 1));
-                __builtin_amdgcn_sched_barrier(0);
-                if (b + 1 < nb) compute(s1);
-                load(s1, min(b + 3, nb - 1));
-                sink(sunk, t2);
-                t2 = touch(min(b + 7, nb - 1));
-                __builtin_amdgcn_sched_barrier(0);
-                if (b + 2 < nb) compute(s0);
-                load(s0, min(b + 4, nb - 1));
-                __builtin_amdgcn_sched_barrier(0);
-                if (b + 3 < nb) compute(s1);
-            }
-            sink(sunk, t0 ^ t2);
-#pragma unroll
-            for (int r = 0; r < RR; ++r)
-                if (po[r] >= 0)
-                    a.h[size_t(po[r]) * a.ff + row] =
-                        silu_mul3(__fmul_rn(0.125f, accg[r]), __fmul_rn(0.125f, accu[r]), a.lim);
-        };
-        __syncthreads();   // the item's scales are staged
-        if (tk.z <= 8) run.template operator()<2>();
-        else run.template operator()<4>();
-    }
-    if (sunk == 0x9e3779b9u && lane == 64) a.h[0] = 0.0f;   // never true (lane < 64): keeps the touches
-}
-
 // IQ2_XS block of the MFMA lane (col, e4) from 16-B parts, as xxs_lane: u[j]
 // holds the 16-bit code (9-bit grid index at bits 7..15, sign bits 0..6) of
 // entry e4 of sub-block 2j (low half) and 2j + 1 (high half).
@@ -509,158 +449,457 @@ __device__ __forceinline__ void xs_lane(const uint4& w, uint32_t (&u)[4]) {
     xpose4(u);
 }
 
-// ---------------------------------------------------------------------------
-// down. Work item = (task, group of NW * 16 output rows; the last group of a
-// task holds what is left of dim, whole waves of 16 rows, and the waves past
-// it only join the item's barriers). IQ2_XS keeps a scale
-// nibble per 16 weights (entries 0, 1 of a sub-block: ls1; entries 2, 3: ls2):
-// per sub-block one MFMA over all 32 weights (C) and one with entries 2, 3 of B
-// zeroed (C1), then ls1 C1 + ls2 (C - C1) as ls2 C + (ls1 - ls2) C1, exactly.
-// ---------------------------------------------------------------------------
-template <int NW, bool TR>
-__global__ __launch_bounds__(NW * 64, 1) void dn_kernel(GroupArgs a) {
-    constexpr int R = NW * 16;   // rows per item
-    constexpr int kL_RS = dn_rs(R);
-    static_assert(dn_lds_bytes(R) <= 160 * 1024, "LDS budget");
-    __shared__ __attribute__((aligned(16))) uint8_t lds[dn_lds_bytes(R)];
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    fill_grid<512, kCopiesXS>(lds, a.tables + kTabXS / 8, t, NW * 64);
-    fill_signs(lds, a.tables, t, NW * 64);
-    __syncthreads();
+// One stream (16 rows) of a tile: where its blocks are. Lane (col, e4) holds row
+// row0 + col; at = that row's first block.
+struct Stream {
+    __amdgpu_buffer_rsrc_t r;
+    uint32_t at;          // row * nb
+    uint32_t o1, o2;      // plane offsets
+};
+// A lane's raw words of one block of one stream: IQ2_XXS q = 16-B part e4 of the
+// row's block; IQ2_XS also s = the block's 8 scale bytes; IQ1_M (from LDS) q.xy = the
+// 8 low index bytes of values 64 e4 .. + 63, q.z their 8 nibbles, s = the scale words.
+struct Raw {
+    uint4 q;
+    uint2 s;
+};
+template <int TY>
+__device__ __forceinline__ void load_raw(Raw& o, const Stream& st, int blk, int e4) {
+    const uint32_t b = st.at + uint32_t(blk);
+    o.q = ld128(st.r, 64u * b + 16u * e4);
+    if constexpr (TY == kIQ2_XS) o.s = ld64(st.r, 8u * b, st.o1);
+}
+// Touches the line of block blk (a row's blocks share a line by twos).
+__device__ __forceinline__ uint32_t touch(const Stream& st, int blk) { return ld32(st.r, 64u * (st.at + uint32_t(blk))); }
+// Four IQ1_M blocks (blk0 .. + 3, past the row's end the last one) of a stream's 16
+// rows, as pieces: row0nb = the stream's first row * nb.
+struct Raw1 {
+    uint4 q[2], h;
+    uint2 s;
+};
+__device__ __forceinline__ void load_raw1(Raw1& o, const Stream& st, uint32_t row0nb, int blk0, int nb, int lane) {
+    const int bq = min(blk0 + ((lane >> 1) & 3), nb - 1), bh = min(blk0 + (lane & 3), nb - 1);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        o.q[i] = ld128(st.r, 32u * (row0nb + uint32_t((8 * i + (lane >> 3)) * nb + bq)) + 16u * (lane & 1));
+    const uint32_t b = row0nb + uint32_t((lane >> 2) * nb + bh);
+    o.h = ld128(st.r, 16u * b, st.o1);
+    o.s = ld64(st.r, 8u * b, st.o2);
+}
+__device__ __forceinline__ void store_raw1(uint8_t* p, const Raw1& o, int lane) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        *reinterpret_cast<uint4*>(p + kR1q * ((lane >> 1) & 3) + 32 * (8 * i + (lane >> 3)) + 16 * (lane & 1)) = o.q[i];
+    *reinterpret_cast<uint4*>(p + kR1ho + kR1h * (lane & 3) + 16 * (lane >> 2)) = o.h;
+    *reinterpret_cast<uint2*>(p + kR1so + kR1s * (lane & 3) + 8 * (lane >> 2)) = o.s;
+}
+__device__ __forceinline__ void read_raw1(Raw& o, const uint8_t* p, int i, int col, int e4) {   // block i of the four
+    const uint2 q = *reinterpret_cast<const uint2*>(p + kR1q * i + 32 * col + 8 * e4);
+    o.q.x = q.x;
+    o.q.y = q.y;
+    o.q.z = *reinterpret_cast<const uint32_t*>(p + kR1ho + kR1h * i + 16 * col + 4 * e4);
+    o.s = *reinterpret_cast<const uint2*>(p + kR1so + kR1s * i + 8 * col);
+}
 
-    const int col = lane & 15, e4 = lane >> 4;
-    const int nb = a.ff / 256, groups = (a.dim + R - 1) / R;
-    const int items = uni(*a.n_tasks) * groups;
-    const uint32_t lo_x = uint32_t(lane & (kCopiesXS - 1)) << 4;        // kL_GRID = 0
-    const uint32_t lo_s = (uint32_t(lane & 31) << 3) | (1u << 16);      // kL_SGN = 1 << 16
-    const uint32_t mk = e4 < 2 ? ~0u : 0u;                               // lanes of entries 0, 1
-    uint32_t sunk = 0;
-    for (int item = blockIdx.x; item < items; item += gridDim.x) {
-        const int task = item / groups, grp = item - task * groups;
-        const int4 tk = task_at(a.tasks, task);
-        const int row0 = grp * R, rows = min(R, a.dim - row0);   // rows: a multiple of 16
-        const int row = row0 + wv * 16 + col;
-        const uint32_t va = uint32_t(slot_off(tk.y, nb, 0, 0, e4) + 16 * col);   // as in gu_kernel
-        int po[4];   // the pairs of the lane's four outputs (tile positions 4 e4 + r)
+// Decoded block of one stream: the MFMA operands of its eight steps and what
+// scales their results. IQ2: step c is sub-block c (32 weights), B its signed
+// grid bytes; XXS: byte c >> 1 of s[c & 1] its factor 2 s + 1; XS: byte c & 3 of
+// s[c >> 2] the factor ls2 of entries 2, 3 and of s[2 + (c >> 2)], signed, ls1 - ls2.
+// IQ1_M: step j is entry j of the lane's 64 values, B scaled; D the factors
+// (2 s + 1) * delta of those entries, in the order of the activations' sums.
+struct Dec {
+    long B[8];
+    uint32_t s[4];
+    long D;
+    float d;   // IQ1_M: the block's fp16 scale
+};
+template <int TY>
+__device__ __forceinline__ void decode(Dec& o, const Raw& w, const uint8_t* lds, int lane, int e4) {
+    if constexpr (TY == kIQ2_XXS) {
+        const uint32_t lo_g = uint32_t(lane & (kCopiesXXS - 1)) << 4;        // kL_GRID = 0
+        const uint32_t lo_s = (uint32_t(lane & 31) << 3) | (1u << 16);       // kL_SGN = 1 << 16
+        const XxsLane X = xxs_lane(w.q, e4);
+        o.s[0] = X.ls[0];
+        o.s[1] = X.ls[1];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int j = 4 * r + e4;
-            po[r] = j < tk.z ? a.order[tk.y + j] : -1;
+        for (int c = 0; c < 8; ++c) {   // grid byte -> address byte 1, then the aux byte
+            const uint32_t u = X.u[c >> 1], h = uint32_t(c & 1) * 2u;
+            const uint4 g = *reinterpret_cast<const uint4*>(lds + perm(u, lo_g, 0x0C020000u | ((4u + h) << 8)));
+            const uint2 m = *reinterpret_cast<const uint2*>(lds + perm(u, lo_s, 0x0C020000u | ((5u + h) << 8)));
+            o.B[c] = pack64(bfi(m.x, g.z, g.x), bfi(m.y, g.w, g.y));
         }
-        const MatRef D = mat_at(a.descs, tk.x, 2);
-        {
-            const uint8_t* planes[1] = {D.base + D.off2};
-            stage_item<NW * 64>(lds, a, tk, a.hd, 1, nb, planes, 1, row0, rows, t, kL_RDD, 0);
-            const int chunks = rows * nb * 8 / 16;   // the rows' IQ2_XS scale bytes
-            for (int i = t; i < chunks; i += NW * 64)
-                *reinterpret_cast<uint4*>(lds + kL_RS + 16 * i) =
-                    reinterpret_cast<const uint4*>(D.base + D.off1 + size_t(row0) * nb * 8)[i];
+    } else if constexpr (TY == kIQ2_XS) {
+        const uint32_t lo_x = uint32_t(lane & (kCopiesXS - 1)) << 4;
+        const uint32_t lo_s = (uint32_t(lane & 31) << 3) | (1u << 16);
+        // Scale byte c holds nibbles lo (entries 0, 1) and hi (entries 2, 3): ls2 =
+        // 2 hi + 1 and ls1 - ls2 = 2 (lo - hi); 128 + 2 lo - 2 hi never borrows.
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t v = h ? w.s.y : w.s.x;
+            const uint32_t hi2 = (v >> 3) & 0x1E1E1E1Eu, lo2 = (v << 1) & 0x1E1E1E1Eu;
+            o.s[h] = hi2 | 0x01010101u;
+            o.s[2 + h] = ((lo2 | 0x80808080u) - hi2) ^ 0x80808080u;
         }
-        const __amdgpu_buffer_rsrc_t rd = rsrc(D.base), rh = rsrc(a.hq);
-        const uint32_t vq = uint32_t(row * nb) * 64u;
-        auto load = [&](DnOps& o, int blk) {
-            o.q = ld128(rd, vq + 64u * blk + 16u * e4);
+        uint32_t u[4];
+        xs_lane(w.q, u);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o.a[i] = ld128(rh, va + 4096u * blk + 1024u * i);
-        };
-        auto touch = [&](int blk) { return ld32(rd, vq + 64u * blk); };
-        // RR: output registers that can hold a pair (ceil(pairs / 4), rounded up to 2, 3 or 4)
-        auto run = [&]<int RR>() {
-            float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            const int rl = wv * 16 + col;   // the lane's row within the item
-            int blk_c = 0;                   // block the next compute() handles
-            auto compute = [&](const DnOps& o) {
-                const int b = blk_c++;
-                const uint2 sc = *reinterpret_cast<const uint2*>(lds + kL_RS + 8 * (rl * nb + b));
-                // Scale byte c holds nibbles lo (entries 0, 1) and hi (entries 2, 3):
-                // ls2 = 2 hi + 1 and ls1 - ls2 = 2 (lo - hi) as byte c & 3 of l2[c >> 2]
-                // and (signed) of dl[c >> 2]; 128 + 2 lo - 2 hi never borrows.
-                uint32_t l2[2], dl[2];
+        for (int c = 0; c < 8; ++c) {
+            const uint32_t v = u[c >> 1], code = (c & 1) ? v >> 16 : v;
+            const uint4 g = *reinterpret_cast<const uint4*>(lds + ((code & 0xff80u) | lo_x));
+            const uint2 m = *reinterpret_cast<const uint2*>(lds + perm(v, lo_s, (c & 1) ? 0x0C020600u : 0x0C020400u));
+            o.B[c] = pack64(bfi(m.x, g.z, g.x), bfi(m.y, g.w, g.y));
+        }
+    } else {
+        // the lane's scale word: s of entries 2k, 2k + 1 at bits 3k; f = those four 2s + 1 as bytes
+        const uint32_t sw = ((e4 & 2) ? w.s.y : w.s.x) >> (16 * (e4 & 1));
+        const uint32_t f = ((sw << 1) & 0xEu) | ((sw << 6) & 0xE00u) | ((sw << 11) & 0xE0000u) | ((sw << 16) & 0xE000000u) | 0x01010101u;
+        const uint32_t nf = ~f + 0x01010101u;   // -(2s + 1) bytewise (f >= 1: no carry)
+        const uint32_t h = w.q.z;   // byte k: nibbles of entries 2k (low) and 2k + 1
+        const uint32_t te = h & 0x07070707u, to = (h >> 4) & 0x07070707u;   // index bits 8..10
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const uint32_t w = h ? sc.y : sc.x;
-                    const uint32_t hi2 = (w >> 3) & 0x1E1E1E1Eu, lo2 = (w << 1) & 0x1E1E1E1Eu;
-                    l2[h] = hi2 | 0x01010101u;
-                    dl[h] = ((lo2 | 0x80808080u) - hi2) ^ 0x80808080u;
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t q = j < 4 ? w.q.x : w.q.y, t = (j & 1) ? to : te;
+            const uint32_t row = perm(t, q, 0x0C0C0000u | uint32_t(j & 3) | ((4u + uint32_t(j >> 1)) << 8));
+            const uint2 g = *reinterpret_cast<const uint2*>(lds + (row << 3));
+            const uint32_t sc = perm(nf, f, 0x0C0C0000u | uint32_t(j >> 1) | ((4u + uint32_t(j >> 1)) << 8));   // 2s + 1, -(2s + 1)
+            o.B[j] = pack64(perm(0u, sc, g.x), perm(0u, sc, g.y));
+        }
+        const uint32_t ne = (h >> 3) & 0x01010101u, no = (h >> 7) & 0x01010101u;   // delta -1
+        const uint32_t me = (ne << 8) - ne, mo = (no << 8) - no;
+        o.D = pack64(bfi(me, nf, f), bfi(mo, nf, f));
+        const uint32_t d16 = ((w.s.x >> 12) & 15u) | ((w.s.x >> 24) & 0xf0u) | ((w.s.y >> 4) & 0xf00u) | ((w.s.y >> 16) & 0xf000u);
+        o.d = h2f(d16);
+    }
+}
+// A block's activations of one tile, a lane's chunk: the four pieces, and IQ1_M's sums.
+template <int TY>
+struct Act {
+    uint4 a[TY == kIQ1_M ? 5 : 4];
+};
+template <int TY>
+__device__ __forceinline__ long act8(const Act<TY>& x, int c) {
+    const uint32_t* av = reinterpret_cast<const uint32_t*>(x.a) + 2 * c;
+    return pack64(av[0], av[1]);
+}
+// Block integers of one IQ1_M stream, bi[r], r < RR: 8 * main + delta, exact.
+template <int RR>
+__device__ __forceinline__ void products1(const Dec& w, const Act<kIQ1_M>& x, int (&bi)[4]) {
+    const v4i L = mfma(act8<kIQ1_M>(x, 8), w.D, v4i{0, 0, 0, 0}), Hs = mfma(act8<kIQ1_M>(x, 9), w.D, v4i{0, 0, 0, 0});
+    v4i M = {0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) M = mfma(act8<kIQ1_M>(x, j), w.B[j], M);
+#pragma unroll
+    for (int r = 0; r < RR; ++r) bi[r] = 8 * M[r] + (16 * Hs[r] + L[r]);
+}
+// Block integers of the two IQ2 streams, bi[s][r], r < RR: exact.
+template <int TY, int RR>
+__device__ __forceinline__ void products(const Dec (&w)[2], const Act<TY>& x, uint32_t mk, int (&bi)[2][4]) {
+    // each step's MFMA is issued before the previous step's multiply-adds read theirs
+    v4i C[16], C1[TY == kIQ2_XS ? 16 : 1];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) bi[0][r] = bi[1][r] = 0;
+#pragma unroll
+    for (int i = 0; i <= 16; ++i) {
+        if (i < 16) {
+            const long A = act8<TY>(x, i >> 1);
+            C[i] = mfma(A, w[i & 1].B[i >> 1], v4i{0, 0, 0, 0});
+            // entries 2, 3 masked out (lanes e4 >= 2 hold them on both sides)
+            if constexpr (TY == kIQ2_XS)
+                C1[i] = mfma(pack64(uint32_t(uint64_t(A)) & mk, uint32_t(uint64_t(A) >> 32) & mk), w[i & 1].B[i >> 1], v4i{0, 0, 0, 0});
+        }
+        if (i > 0) {
+            const int s = (i - 1) & 1, c = (i - 1) >> 1;
+            if constexpr (TY == kIQ2_XS) {   // ls1 C1 + ls2 (C - C1) as ls2 C + (ls1 - ls2) C1, exactly
+                const int ls2 = int(__builtin_amdgcn_ubfe(w[s].s[c >> 2], 8 * (c & 3), 8));
+                const int dls = __builtin_amdgcn_sbfe(int(w[s].s[2 + (c >> 2)]), 8 * (c & 3), 8);
+#pragma unroll
+                for (int r = 0; r < RR; ++r) bi[s][r] = mad24(ls2, C[i - 1][r], mad24(dls, C1[i - 1][r], bi[s][r]));
+            } else {
+                const int ls = int(__builtin_amdgcn_ubfe(w[s].s[c & 1], 8 * (c >> 1), 8));
+#pragma unroll
+                for (int r = 0; r < RR; ++r) bi[s][r] = mad24(ls, C[i - 1][r], bi[s][r]);
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Tiles. GU: rows 16 tl .. + 15 of gate and of up; down: rows 32 tl .. + 31.
+// ---------------------------------------------------------------------------
+// LDS written by one wave and read by its other lanes.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+// TR: also write each pair's block integers (GroupArgs::tint).
+template <bool GU, int TY, bool TR, bool DB>
+__device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int tl, uint8_t* lds, uint8_t* wl, int lane,
+                                        uint32_t& sunk) {
+    const int col = lane & 15, e4 = lane >> 4, nb = (GU ? a.dim : a.ff) / 256;
+    const uint32_t mk = e4 < 2 ? ~0u : 0u;   // lanes of entries 0, 1
+    Stream st[2];
+    const uint8_t* planes[2];   // fp16 scales of the streams' rows
+    if constexpr (GU) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const MatRef m = mat_at(a.descs, tk.x, s);
+            st[s] = Stream{rsrc(m.base), uint32_t(16 * tl + col) * uint32_t(nb), uint32_t(m.off1), uint32_t(m.off2)};
+            planes[s] = m.base + (TY == kIQ2_XXS ? m.off1 : m.off2) + size_t(16 * tl) * nb * 2;
+        }
+    } else {
+        const MatRef m = mat_at(a.descs, tk.x, 2);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            st[s] = Stream{rsrc(m.base), uint32_t(32 * tl + 16 * s + col) * uint32_t(nb), uint32_t(m.off1), uint32_t(m.off2)};
+            planes[s] = m.base + (TY == kIQ2_XXS ? m.off1 : m.off2) + size_t(32 * tl + 16 * s) * nb * 2;
+        }
+    }
+    // A operand: slot col of the tile (past its pairs: unused slot memory, whose
+    // outputs are discarded), the lane's chunk e4
+    const __amdgpu_buffer_rsrc_t rx = rsrc((GU ? a.xq : a.hq) + tile_off(tk.y >> 4, nb));
+    const uint32_t va = 256u * e4 + 16u * col;
+    Act<TY> x0, x1;
+    auto load_x = [&](Act<TY>& x, int blk) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x.a[i] = ld128(rx, va + 4096u * blk + 1024u * i);
+        if constexpr (TY == kIQ1_M) x.a[4] = ld128(rx, va + 1024u * blk, 4096u * nb);
+    };
+    Raw w0[2], w1[2];   // IQ2
+    uint32_t t0 = 0, t2 = 0;
+    auto load = [&](Raw (&w)[2], Act<TY>& x, int blk) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) load_raw<TY>(w[s], st[s], blk, e4);
+        load_x(x, blk);
+    };
+    auto touch2 = [&](int blk) { return touch(st[0], blk) ^ touch(st[1], blk); };
+    Raw1 r1[2];         // IQ1_M
+    const uint32_t row0nb[2] = {uint32_t(GU ? 16 * tl : 32 * tl) * uint32_t(nb), uint32_t(GU ? 16 * tl : 32 * tl + 16) * uint32_t(nb)};
+    if constexpr (TY == kIQ1_M) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) load_raw1(r1[s], st[s], row0nb[s], 0, nb, lane);
+        if (DB) load_x(x0, 0);
+    } else {
+        load(w0, x0, 0);
+        t0 = touch2(min(1, nb - 1));
+        t2 = touch2(min(3, nb - 1));
+    }
+    // the tile's pair scales and rows' scales into the wave's own LDS
+    float* pd = reinterpret_cast<float*>(wl);
+    uint16_t* rd = reinterpret_cast<uint16_t*>(wl + 64 * kGrpNb);
+    const float4* pds = reinterpret_cast<const float4*>((GU ? a.xd : a.hd) + size_t(tk.y >> 4) * nb * 16);
+    wave_sync();   // the previous tile's are read
+    for (int i = lane; i < 4 * nb; i += 64) reinterpret_cast<float4*>(pd)[i] = pds[i];
+    if constexpr (TY != kIQ1_M) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+            for (int i = lane; i < 2 * nb; i += 64)   // 16 rows x nb halves, 16 B a piece
+                reinterpret_cast<uint4*>(rd + 16 * kGrpNb * s)[i] = reinterpret_cast<const uint4*>(planes[s])[i];
+    }
+    int po[4];   // the pairs of the lane's four outputs (tile positions 4 e4 + r)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int j = 4 * r + e4;
+        po[r] = j < tk.z ? a.order[tk.y + j] : -1;
+    }
+    wave_sync();
+    // RR: output registers that can hold a pair (ceil(pairs / 4), rounded up to 2 or 4)
+    auto run = [&]<int RR>() {
+        float acc[2][4] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+        int blk_c = 0;   // block the next compute() handles
+        auto compute = [&](const Raw (&w)[2], const Act<TY>& x) {
+            const int b = blk_c++;
+            Dec dec[2];
+            int bi[2][4];
+            if constexpr (TY == kIQ1_M) {
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {   // one stream after the other: both at once spill
+                    decode<TY>(dec[s], w[s], lds, lane, e4);
+                    products1<RR>(dec[s], x, bi[s]);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-                int bi[4] = {0, 0, 0, 0};
-                uint32_t u[4];
-                xs_lane(o.q, u);
-                uint4 g[8];
-                uint2 m[8];
+            } else {
 #pragma unroll
-                for (int c = 0; c < 8; ++c) {   // all eight lookups in flight before the first use
-                    const uint32_t w = u[c >> 1], code = (c & 1) ? w >> 16 : w;
-                    g[c] = *reinterpret_cast<const uint4*>(lds + ((code & 0xff80u) | lo_x));
-                    m[c] = *reinterpret_cast<const uint2*>(lds + perm(w, lo_s, (c & 1) ? 0x0C020600u : 0x0C020400u));
-                }
-                // sub-block c's two MFMAs are issued before sub-block c - 1's scale
-                // multiply-adds read their results (no wait states between them)
-                v4i C[8], C1[8];
+                for (int s = 0; s < 2; ++s) decode<TY>(dec[s], w[s], lds, lane, e4);
+                products<TY, RR>(dec, x, mk, bi);
+            }
+            if constexpr (TR) {   // pair po[r]'s block integers of this lane's rows
+                const size_t gu = size_t(a.ff) * (a.dim / 256), rec = 2 * gu + size_t(a.dim) * (a.ff / 256);
 #pragma unroll
-                for (int c = 0; c <= 8; ++c) {
-                    if (c < 8) {
-                        const uint32_t* av = reinterpret_cast<const uint32_t*>(o.a) + 2 * c;
-                        const long A = pack64(av[0], av[1]);
-                        const uint32_t blo = bfi(m[c].x, g[c].z, g[c].x), bhi = bfi(m[c].y, g[c].w, g[c].y);
-                        C[c] = mfma(A, pack64(blo, bhi), v4i{0, 0, 0, 0});
-                        C1[c] = mfma(A, pack64(blo & mk, bhi & mk), v4i{0, 0, 0, 0});
-                    }
-                    if (c > 0) {
-                        const int p = c - 1;
-                        const int ls2 = int(__builtin_amdgcn_ubfe(l2[p >> 2], 8 * (p & 3), 8));
-                        const int dls = __builtin_amdgcn_sbfe(int(dl[p >> 2]), 8 * (p & 3), 8);
-#pragma unroll
-                        for (int r = 0; r < RR; ++r) bi[r] = mad24(ls2, C[p][r], mad24(dls, C1[p][r], bi[r]));
-                    }
-                }
-                if constexpr (TR) {
-                    const int nbx = a.dim / 256;
-                    const size_t rec = 2 * size_t(a.ff) * nbx + size_t(a.dim) * nb;
+                for (int s = 0; s < 2; ++s)
 #pragma unroll
                     for (int r = 0; r < RR; ++r)
                         if (a.tint && po[r] >= 0)
-                            a.tint[size_t(po[r]) * rec + 2 * size_t(a.ff) * nbx + size_t(row) * nb + size_t(b)] = bi[r];
-                }
-                const float ddf = h2f(reinterpret_cast<const uint16_t*>(lds + kL_RDD)[rl * nb + b]);
-                const float4 hd4 = *reinterpret_cast<const float4*>(lds + kL_PD + 64 * b + 16 * e4);
-                const float hd[4] = {hd4.x, hd4.y, hd4.z, hd4.w};
+                            a.tint[size_t(po[r]) * rec + (GU ? s * gu : 2 * gu) + st[s].at + size_t(b)] = bi[s][r];
+            }
+            const float4 xd4 = *reinterpret_cast<const float4*>(pd + 16 * b + 4 * e4);
+            const float xd[4] = {xd4.x, xd4.y, xd4.z, xd4.w};
 #pragma unroll
-                for (int r = 0; r < RR; ++r) acc[r] = fmaf(__fmul_rn(ddf, hd[r]), float(bi[r]), acc[r]);
-            };
-            DnOps s0, s1;
-            load(s0, 0);
-            uint32_t t0 = touch(min(1, nb - 1)), t2 = touch(min(3, nb - 1));
+            for (int s = 0; s < 2; ++s) {
+                const float d = TY == kIQ1_M ? dec[s].d : h2f(rd[16 * kGrpNb * s + col * nb + b]);
+#pragma unroll
+                for (int r = 0; r < RR; ++r) acc[s][r] = fmaf(__fmul_rn(d, xd[r]), float(bi[s][r]), acc[s][r]);
+            }
+        };
+        if constexpr (TY == kIQ1_M) {
+            // four blocks at a time through the wave's LDS, the next four in registers
+            // meanwhile
+            uint8_t* raw = wl + 64 * kGrpNb;
             for (int b = 0; b < nb; b += 4) {
-                load(s1, min(b + 1, nb - 1));
+                wave_sync();   // the previous four are read
+#pragma unroll
+                for (int s = 0; s < 2; ++s) store_raw1(raw + kRaw1 * s, r1[s], lane);
+                wave_sync();
+#pragma unroll
+                for (int s = 0; s < 2; ++s) load_raw1(r1[s], st[s], row0nb[s], min(b + 4, nb - 1), nb, lane);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    Act<TY>& now = DB && (i & 1) ? x1 : x0;
+                    Act<TY>& then = DB && !(i & 1) ? x1 : x0;
+                    if (DB) load_x(then, min(b + i + 1, nb - 1));
+                    if (b + i < nb) {
+                        if (!DB) load_x(now, b + i);   // under the first stream's decode (a second set spills)
+                        __builtin_amdgcn_sched_barrier(0);
+                        Raw w[2];
+#pragma unroll
+                        for (int s = 0; s < 2; ++s) read_raw1(w[s], raw + kRaw1 * s, i, col, e4);
+                        compute(w, now);
+                    }
+                }
+            }
+        } else {
+            // Two operand sets alternate over a 4-step unrolled loop (no register copies,
+            // so no wait ever covers a load issued in the same step); line touches four
+            // blocks ahead in fixed registers, one per line of two blocks.
+            for (int b = 0; b < nb; b += 4) {
+                load(w1, x1, min(b + 1, nb - 1));
                 sink(sunk, t0);
-                t0 = touch(min(b + 5, nb - 1));
+                t0 = touch2(min(b + 5, nb - 1));
                 __builtin_amdgcn_sched_barrier(0);   // the loads stay ahead of the compute
-                compute(s0);
-                load(s0, min(b + 2, nb - 1));
+                compute(w0, x0);
+                load(w0, x0, min(b + 2, nb - 1));
                 __builtin_amdgcn_sched_barrier(0);
-                if (b + 1 < nb) compute(s1);
-                load(s1, min(b + 3, nb - 1));
+                if (b + 1 < nb) compute(w1, x1);
+                load(w1, x1, min(b + 3, nb - 1));
                 sink(sunk, t2);
-                t2 = touch(min(b + 7, nb - 1));
+                t2 = touch2(min(b + 7, nb - 1));
                 __builtin_amdgcn_sched_barrier(0);
-                if (b + 2 < nb) compute(s0);
-                load(s0, min(b + 4, nb - 1));
+                if (b + 2 < nb) compute(w0, x0);
+                load(w0, x0, min(b + 4, nb - 1));
                 __builtin_amdgcn_sched_barrier(0);
-                if (b + 3 < nb) compute(s1);
+                if (b + 3 < nb) compute(w1, x1);
             }
             sink(sunk, t0 ^ t2);
+        }
 #pragma unroll
-            for (int r = 0; r < RR; ++r)
-                if (po[r] >= 0) a.y[size_t(po[r]) * a.dim + row] = __fmul_rn(0.125f, acc[r]);
-        };
-        __syncthreads();   // the item's scales are staged
-        if (wv * 16 >= rows) continue;   // wave-uniform: no rows of this wave in the last group
-        if (tk.z <= 8) run.template operator()<2>();
-        else if (tk.z <= 12) run.template operator()<3>();
-        else run.template operator()<4>();
+        for (int r = 0; r < RR; ++r)
+            if (po[r] >= 0) {
+                if constexpr (GU) {
+                    a.h[size_t(po[r]) * a.ff + 16 * tl + col] =
+                        silu_mul3(__fmul_rn(0.125f, acc[0][r]), __fmul_rn(0.125f, acc[1][r]), a.lim);
+                } else {
+                    float* y = a.y + size_t(po[r]) * a.dim + 32 * tl + col;
+                    y[0] = __fmul_rn(0.125f, acc[0][r]);
+                    y[16] = __fmul_rn(0.125f, acc[1][r]);
+                }
+            }
+    };
+    if (tk.z <= 8) run.template operator()<2>();
+    else run.template operator()<4>();
+}
+
+// MASK: block types among the launch's matrices (bits 1 IQ2_XXS, 2 IQ2_XS, 4 IQ1_M).
+template <bool GU, int MASK, int NW, bool TR>
+__global__ __launch_bounds__(NW * 64, 1) void grouped_kernel(GroupArgs a) {
+    __shared__ __attribute__((aligned(16))) uint8_t lds[grp_lds_bytes(MASK, NW)];
+    __shared__ uint32_t s_bundle;   // current bundle << 8 | its next tile
+    __shared__ int s_open;
+    const int t = threadIdx.x, lane = t & 63, wv = uni(t >> 6);
+    const int tiles = GU ? a.ff / 16 : a.dim / 32;   // per task
+    int n[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) n[i] = uni(GU ? a.queue->gu_tasks[i] : a.queue->dn_tasks[i]);
+    int* next = GU ? a.queue->gu_next : a.queue->dn_next;
+    // the type this workgroup starts with: its place in the tasks weighted by their cost
+    int first = 0;
+    if constexpr (MASK == 7) {
+        const int c0 = kTileCost[0] * n[0], c1 = c0 + kTileCost[1] * n[1], all = c1 + kTileCost[2] * n[2];
+        const int64_t at = int64_t(all) * (2 * blockIdx.x + 1);
+        first = at < int64_t(c0) * 2 * gridDim.x ? 0 : at < int64_t(c1) * 2 * gridDim.x ? 1 : 2;
     }
-    if (sunk == 0x9e3779b9u && lane == 64) a.y[0] = 0.0f;   // never true (lane < 64): keeps the touches
+    uint32_t sunk = 0;
+    for (int i = 0; i < (MASK == 7 ? 3 : 1); ++i) {
+        const int ti = MASK == 7 ? (first + i) % 3 : MASK == 1 ? 0 : MASK == 2 ? 1 : 2;
+        const int base = ti == 0 ? 0 : ti == 1 ? n[0] : n[0] + n[1];   // the type's tasks in the list
+        const int total = n[ti] * tiles;
+        // tiles per bundle: a workgroup's waves on one task's activations, or fewer
+        // where that would leave the last round of bundles short
+        // (few tiles of one type: an even share each, no queue)
+        const bool even = MASK != 7 && total <= 2 * NW * int(gridDim.x);
+        const int start = even ? int(int64_t(total) * blockIdx.x / gridDim.x) : 0;
+        const int bs = even ? int(int64_t(total) * (blockIdx.x + 1) / gridDim.x) - start
+                            : total >= 16 * NW * int(gridDim.x) ? NW : 4;
+        uint8_t* wl = ti == 2 ? lds + kL_TAB1 + wv * kL_WAVE1 : lds + kL_TAB + wv * kL_WAVE;
+        if (MASK == 7 || i == 0) {
+            __syncthreads();   // every wave is done with the previous type's tables
+            if (t == 0) {
+                s_open = total > 0 && (i == 0 || __hip_atomic_load(next + ti, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * bs < total);
+                // one type: the first bundle is the workgroup's own; several: none yet
+                s_bundle = even ? 0u : MASK != 7 ? uint32_t(blockIdx.x) << 8 : uint32_t(bs);
+            }
+            __syncthreads();
+        }
+        if (!s_open) continue;   // nothing left of this type (workgroup-uniform)
+        uint32_t warm[2] = {0, 0};
+        if (MASK != 7) {   // the chain of loads to the wave's first rows, under the tables' fill
+            const int ft = even ? start + wv : int(blockIdx.x) * bs + wv;
+            if (bs == 0) break;
+            if (wv < bs && ft < total) {
+                const int task = ft / tiles, tl = ft - task * tiles, nb = (GU ? a.dim : a.ff) / 256;
+                const int4 tk = task_at((GU ? a.tasks : a.dtasks) + base, task);
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const MatRef m = mat_at(a.descs, tk.x, GU ? s : 2);
+                    const int row = (GU ? 16 * tl : 32 * tl + 16 * s) + (lane & 15);
+                    warm[s] = ld32(rsrc(m.base), (ti == 2 ? 32u : 64u) * uint32_t(row * nb));
+                }
+            }
+        }
+        fill_tables<NW * 64>(lds, ti == 0 ? kIQ2_XXS : ti == 1 ? kIQ2_XS : kIQ1_M, a.tables, t);
+        __syncthreads();
+        sink(sunk, warm[0] ^ warm[1]);
+        for (;;) {
+            uint32_t got = 0;
+            for (;;) {   // this wave's next tile
+                if (lane == 0) got = atomicAdd(&s_bundle, 1u);
+                got = uint32_t(uni(int(got)));
+                const uint32_t at = got & 255u;
+                if (at < uint32_t(bs) || even) break;
+                if (at == uint32_t(bs)) {   // empty: this wave fetches the next bundle and takes its first tile
+                    int b = 0;
+                    if (lane == 0) b = atomicAdd(next + ti, 1);
+                    b = min(uni(b), (total + bs - 1) / bs);   // past the last: an empty bundle that ends every wave
+                    got = uint32_t(b) << 8;
+                    if (lane == 0) __hip_atomic_store(&s_bundle, got | 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    break;
+                }
+                // Past bs: another wave is fetching one (it waits for nothing but the queue's
+                // atomic). At bs itself nobody is: a wave that missed a whole bundle
+                // between two looks must draw again, or, with every other wave gone
+                // after the last bundle, it would wait for good.
+                while ((__hip_atomic_load(&s_bundle, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & 255u) > uint32_t(bs))
+                    __builtin_amdgcn_s_sleep(1);
+            }
+            if (even && got >= uint32_t(bs)) break;
+            const int tile = even ? start + int(got) : int(got >> 8) * bs + int(got & 255u);
+            if (tile >= total) break;
+            const int task = tile / tiles, tl = tile - task * tiles;
+            const int4 tk = task_at((GU ? a.tasks : a.dtasks) + base, task);
+            if (MASK == 1 || (MASK == 7 && ti == 0)) do_tile<GU, kIQ2_XXS, TR, NW <= 8>(a, tk, tl, lds, wl, lane, sunk);
+            else if (MASK == 2 || (MASK == 7 && ti == 1)) do_tile<GU, kIQ2_XS, TR, NW <= 8>(a, tk, tl, lds, wl, lane, sunk);
+            else do_tile<GU, kIQ1_M, TR, NW <= 8>(a, tk, tl, lds, wl, lane, sunk);
+        }
+    }
+    if (sunk == 0x9e3779b9u && lane == 64) (GU ? a.h : a.y)[0] = 0.0f;   // never true (lane < 64): keeps the touches
 }
 
 // ---------------------------------------------------------------------------
@@ -719,37 +958,40 @@ __global__ __launch_bounds__(256) void gcombine_kernel(GroupArgs a) {
 
 }  // namespace
 
-hipError_t launch_grouped(const GroupArgs& args, int cus, hipStream_t s) {
-    // gate/up: 12 waves per workgroup (3 per SIMD, 192 rows per item) where ff
-    // allows, else 8; down: 12 (its last group of a task ragged)
-    constexpr int NW = 8, NWD = 12;
-    if (args.T < 1 || args.k < 1 || args.k > 16 || args.n_experts > kGroupMaxExperts || args.dim % (NW * 16) ||
-        args.ff % (NW * 16) || args.dim % 256 || args.ff % 256 || args.dim > kGuNb * 256 || args.ff > kDnNb * 256)
+hipError_t launch_grouped(GroupArgs args, int gu_types, int dn_types, int cus, hipStream_t s) {
+    // waves per workgroup: 3 per SIMD; layers of several types 2, whose kernel spills
+    // 50 registers at 3 (512 tokens, 4096 x 3072, 384 experts: 1,426 against 1,494 us)
+    constexpr int NW = 12, NWM = 8;
+    if (args.T < 1 || args.k < 1 || args.k > 16 || args.n_experts > kGroupMaxExperts || args.dim % 256 || args.ff % 256 ||
+        args.dim > kGrpNb * 256 || args.ff > 4096 || args.cap < kTile || args.cap % kTile)
         return hipErrorNotSupported;
-    const bool gu12 = args.ff % (12 * 16) == 0;
-    const int P = args.T * args.k;
+    const bool trace = args.tq8x || args.tq8h || args.th || args.tint;
+    if (trace && (gu_types != 1 || dn_types != 2)) return hipErrorNotSupported;
+    const int P = args.T * args.k, nbx = args.dim / 256, nbh = args.ff / 256;
+    const auto grouped = [&](auto kernel, int nw = 12) { hipLaunchKernelGGL(kernel, dim3(cus), dim3(nw * 64), 0, s, args); };
+    const auto rows = [&](auto kernel, const float* src, int n, int nb, int8_t* q, float* d, uint8_t* tr) {
+        hipLaunchKernelGGL(kernel, dim3((n * nb + 3) / 4), dim3(256), 0, s, src, n, nb, q, d, args.pos, args.k, args.err, tr);
+    };
+    // the queues start past the workgroups' own first bundles (launches of one type)
+    args.gu_first = gu_types == 1 || gu_types == 4 ? cus : 0;
+    args.dn_first = dn_types == 2 || dn_types == 4 ? cus : 0;
     hipLaunchKernelGGL(bucket_kernel, dim3(1), dim3(1024), 0, s, args);
-    const int nbx = args.dim / 256, nbh = args.ff / 256;
-    if (args.tq8x || args.tq8h || args.th || args.tint) {   // the parity trace (separate instances)
-        hipLaunchKernelGGL((q8k_rows_kernel<ROWS_X, true>), dim3((args.T * nbx + 3) / 4), dim3(256), 0, s, args.x,
-                           args.T, nbx, args.xq, args.xd, args.pos, args.k, args.err, args.tq8x);
-        if (gu12)
-            hipLaunchKernelGGL((gu_kernel<12, true>), dim3(cus), dim3(12 * 64), 0, s, args);
-        else
-            hipLaunchKernelGGL((gu_kernel<NW, true>), dim3(cus), dim3(NW * 64), 0, s, args);
-        hipLaunchKernelGGL((q8k_rows_kernel<ROWS_H, true>), dim3((P * nbh + 3) / 4), dim3(256), 0, s, args.h, P, nbh,
-                           args.hq, args.hd, args.pos, args.k, args.err, args.tq8h);
-        hipLaunchKernelGGL((dn_kernel<NWD, true>), dim3(cus), dim3(NWD * 64), 0, s, args);
+    if (trace) {   // the parity trace (separate instances)
+        rows((q8k_rows_kernel<ROWS_X, false, true>), args.x, args.T, nbx, args.xq, args.xd, args.tq8x);
+        grouped(grouped_kernel<true, 1, NW, true>);
+        rows((q8k_rows_kernel<ROWS_H, false, true>), args.h, P, nbh, args.hq, args.hd, args.tq8h);
+        grouped(grouped_kernel<false, 2, NW, true>);
     } else {
-        hipLaunchKernelGGL((q8k_rows_kernel<ROWS_X, false>), dim3((args.T * nbx + 3) / 4), dim3(256), 0, s, args.x,
-                           args.T, nbx, args.xq, args.xd, args.pos, args.k, args.err, nullptr);
-        if (gu12)
-            hipLaunchKernelGGL((gu_kernel<12, false>), dim3(cus), dim3(12 * 64), 0, s, args);
-        else
-            hipLaunchKernelGGL((gu_kernel<NW, false>), dim3(cus), dim3(NW * 64), 0, s, args);
-        hipLaunchKernelGGL((q8k_rows_kernel<ROWS_H, false>), dim3((P * nbh + 3) / 4), dim3(256), 0, s, args.h, P, nbh,
-                           args.hq, args.hd, args.pos, args.k, args.err, nullptr);
-        hipLaunchKernelGGL((dn_kernel<NWD, false>), dim3(cus), dim3(NWD * 64), 0, s, args);
+        rows(gu_types & 4 ? q8k_rows_kernel<ROWS_X, true, false> : q8k_rows_kernel<ROWS_X, false, false>, args.x, args.T, nbx,
+             args.xq, args.xd, nullptr);
+        if (gu_types == 1) grouped(grouped_kernel<true, 1, NW, false>);
+        else if (gu_types == 4) grouped(grouped_kernel<true, 4, NW, false>);
+        else grouped(grouped_kernel<true, 7, NWM, false>, NWM);
+        rows(dn_types & 4 ? q8k_rows_kernel<ROWS_H, true, false> : q8k_rows_kernel<ROWS_H, false, false>, args.h, P, nbh,
+             args.hq, args.hd, nullptr);
+        if (dn_types == 2) grouped(grouped_kernel<false, 2, NW, false>);
+        else if (dn_types == 4) grouped(grouped_kernel<false, 4, NW, false>);
+        else grouped(grouped_kernel<false, 7, NWM, false>, NWM);
     }
     const bool al16 = (reinterpret_cast<uintptr_t>(args.out) | reinterpret_cast<uintptr_t>(args.shared)) % 16 == 0;
     if (al16) hipLaunchKernelGGL(gcombine_kernel<4>, dim3((args.dim / 4 + 255) / 256, args.T), dim3(256), 0, s, args);

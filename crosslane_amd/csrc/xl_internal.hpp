@@ -114,6 +114,11 @@ struct Layer3Args {
 constexpr int kHBufWords = 16 * 4096;      // k_max * ff_max
 constexpr int kStreamRouteMax = 512;       // experts a streaming kernel routes itself (8 per lane)
 
+// Per block type (IQ2_XXS, IQ2_XS, IQ1_M): the tasks whose gate / down matrices
+// have it, and the next bundle of their tiles to hand out.
+struct GroupQueue {
+    int gu_tasks[3], dn_tasks[3], gu_next[3], dn_next[3];
+};
 // Arguments of the grouped path (xl_grouped.hip): T tokens with k picks each,
 // P = T * k (token, pick) pairs, pair p = token p / k. Device pointers.
 struct GroupArgs {
@@ -124,14 +129,17 @@ struct GroupArgs {
     const float* shared;        // T * dim, or null
     float* out;                 // T * dim
     int T, k, n_experts, dim, ff;
-    // Slots: task i owns slots 16 i .. 16 i + 15, its pairs in the first ones.
-    int8_t* xq; float* xd;      // Q8_K(x): quants per slot (16 * max tasks * dim, the MFMA order), scales per token
-    int32_t* order;             // pair of each used slot (16 * max tasks)
-    int32_t* pos;               // slot of each pair (P; -1 for a bad id)
-    int4* tasks;                // (expert, first slot, pairs <= 16, 0) per task
-    int32_t* n_tasks;           // tasks written by the bucket kernel
+    // Slots: tile i of 16 pairs owns slots 16 i .. 16 i + 15; a task is up to cap
+    // pairs of one expert (cap a multiple of 16), in consecutive tiles.
+    int8_t* xq; float* xd;      // Q8_K(x): quants per tile (5/4 * 16 * dim bytes each, the MFMA order), scales per slot
+    int32_t* order;             // pair of each used slot (16 * max tiles)
+    int32_t* pos;               // slot of each pair (P; -1 for a bad id), with order bits (xl_grouped.hip)
+    int4* tasks; int4* dtasks;  // (expert, first slot, pairs, 0) per task, by gate type and by down type
+    GroupQueue* queue;          // task counts and work queues, written by the bucket kernel
+    int cap;
+    int gu_first, dn_first;     // the queues' first bundles (set by launch_grouped)
     float* h;                   // P * ff
-    int8_t* hq; float* hd;      // Q8_K(h): quants per slot (16 * max tasks * ff), scales per pair
+    int8_t* hq; float* hd;      // Q8_K(h): as xq and xd, of ff
     float* y;                   // P * dim
     const uint64_t* tables;     // expanded codebooks (kLayer3TableBytes)
     int* err;
@@ -145,10 +153,16 @@ struct GroupArgs {
     float* th;
     int32_t* tint;
 };
+// Tokens from which layers that are not IQ2_XXS gate/up + IQ2_XS down run grouped.
+// Measured at 4096 x 3072, 384 experts, 6 picks: 13 tokens 327 us (mixed types) and
+// 265 us (IQ1_M) grouped against 354 and 298 us by layer calls, about level at 12
+// (fewer experts or smaller shapes gain earlier: 13 tokens at 1024 x 512 take 41 us
+// against 158). Below it a call keeps the bits of its tokens' single layer calls.
+constexpr int kGroupAnyTokens = 13;
 constexpr int kGroupMaxExperts = 8192;
 constexpr int kRouteMaxExperts = 4096;   // router: scores and keys of one token in LDS   // experts per layer the bucket kernel counts in LDS
-// Tasks the bucket kernel can write for P pairs: one per started tile of 16 pairs of an expert.
-inline int64_t group_max_tasks(int64_t P, int64_t n_experts) { return P / 16 + (P < n_experts ? P : n_experts) + 1; }
+// Tiles (and at most as many tasks) for P pairs: one per started 16 pairs of an expert.
+inline int64_t group_max_tiles(int64_t P, int64_t n_experts) { return P / 16 + (P < n_experts ? P : n_experts) + 1; }
 constexpr int kLayer3TableBytes = 24576;   // expanded codebooks of the single-launch kernel
 // Then the IQ1_M value rows of the streaming kernels: 4096 rows of 8 int8,
 // row (nib << 8 | idx_lo) = 8 * grid[(nib & 7) << 8 | idx_lo] + (nib & 8 ? -1 : 1).
@@ -176,9 +190,10 @@ hipError_t launch_stream(const Layer3Args& args, int gu_types, int dn_types, int
                          hipEvent_t stop = nullptr);
 hipError_t launch_stream_iq1(const Layer3Args& args, int cus, hipStream_t s, hipEvent_t stop);
 hipError_t launch_stream_mix(const Layer3Args& args, int cus, hipStream_t s, hipEvent_t stop);
-// Grouped path: hipErrorNotSupported unless gate/up are IQ2_XXS, down IQ2_XS and
-// the shapes fit (dim, ff multiples of 128; n_experts <= kGroupMaxExperts).
-hipError_t launch_grouped(const GroupArgs& args, int cus, hipStream_t s);
+// Grouped path (gu_types / dn_types: as launch_layer3): hipErrorNotSupported unless
+// the shapes fit (dim, ff multiples of 256 up to 5120 / 4096; n_experts <=
+// kGroupMaxExperts); traced, unless gate/up are IQ2_XXS and down IQ2_XS.
+hipError_t launch_grouped(GroupArgs args, int gu_types, int dn_types, int cus, hipStream_t s);
 hipError_t launch_q8k(const float* x, int nblocks, int8_t* qs, float* d, uint8_t* std_out, int* err, hipStream_t s);
 // Rows in the reference CPU lane's float order (xl_exact.hip): role 0 gives
 // h = SwiGLU(gate . a, up . a) of every pick (out: k x rows), role 2 the down

@@ -63,7 +63,7 @@ typedef struct xl_config {
     int32_t max_picks;     /* top-k bound, 1..16 (reference kPicks = 8, model_meta.hpp:18) */
     int32_t max_tokens;    /* grouped-path token bound (0 = grouped path unused). Its
                               workspace, with P = max_tokens * max_picks: about
-                              16 * (P / 16 + min(P, n_experts) + 1) * (dim + ff) bytes
+                              20 * (P / 16 + min(P, n_experts) + 1) * (dim + ff) bytes
                               of per-slot quants plus 4 * P * (dim + ff) bytes of h
                               and per-pick rows (~200 MB at 512 tokens, 8 picks,
                               384 experts, 4096 x 3072) */
@@ -168,8 +168,8 @@ int32_t xl_sync(xl_context* ctx, void* stream, xl_error* err);
  * token: WarmRedirect::warm_compute_many, engine/strata/warm/runtime.hpp:13,
  * then warm_execute's fixed-order combine, runtime.cpp:180-188), with every
  * touched expert's weights read once per 16 of its (token, pick) pairs on
- * int8 MFMA for IQ2_XXS gate/up + IQ2_XS down layers (other layers run one
- * layer call per token). Needs a context opened with max_tokens >= T; picks
+ * int8 MFMA: IQ2_XXS gate/up + IQ2_XS down layers always, layers of other or
+ * mixed types from 13 tokens on (below, one layer call per token). Needs a context opened with max_tokens >= T; picks
  * of one token unique. The async form takes device pointers and checks ids on
  * the device (a bad id sets the flag; that pick contributes nothing). */
 int32_t xl_grouped_forward(xl_context* ctx, int32_t layer, int32_t T, int32_t k, const int32_t* ids, const float* w,
