@@ -1128,7 +1128,7 @@ void enqueue_grouped(xl_context* ctx, int32_t layer, int32_t T, int32_t k, const
         a.T = T; a.k = k; a.n_experts = E; a.dim = dim; a.ff = ctx->cfg.ff;
         const auto& g = ctx->grp;
         a.xq = g.xq; a.xd = g.xd; a.order = g.order; a.pos = g.pos; a.tasks = g.tasks; a.dtasks = g.dtasks;
-        a.queue = g.queue; a.cap = 16;
+        a.queue = g.queue;
         a.h = g.h; a.hq = g.hq; a.hd = g.hd; a.y = g.y;
         a.tables = ctx->tables; a.err = ctx->err_flag;
         a.lim = ctx->cfg.swiglu_limit;

@@ -59,6 +59,7 @@
 // IQ1_M 1,265, mixed types 1,426 (10,999 and 12,992 as 512 layer calls).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "xl_dev.hpp"
@@ -73,6 +74,12 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 constexpr int kTile = 16;   // pairs per tile (the MFMA M dimension)
 // GroupArgs::pos: slot of a pair, and whether its x / h go there in the IQ1_M order.
 constexpr int kSlotX1 = 1 << 30, kSlotH1 = 1 << 29, kSlotMask = kSlotH1 - 1;
+// Pairs per expert from which tasks hold up to 64 pairs, in kernels of 8 waves (2 per
+// SIMD: their registers). 4096 x 3072, 384 experts, IQ2: 12 per expert 1,582 us, 32
+// per expert 2,341 us (3,075 by 16-pair tasks); 11 per expert 1,587 against 1,548, 8
+// per expert 1,528 against 1,449. Also where a workgroup has at most 8 tiles: 12 waves
+// would share them (1024 x 512, 64 experts, 64 tokens: 46.0 against 51.8 us).
+constexpr int kMultiPairs = 12;
 // Relative cost of a tile by type (XXS, XS, IQ1_M), for the first share of a mixed
 // layer's workgroups (the queues even out what it misses).
 __device__ constexpr int kTileCost[3] = {10, 11, 8};
@@ -807,8 +814,158 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
     else run.template operator()<4>();
 }
 
+// A tile of a task of 16 (NT - 1) + 1 .. 16 NT pairs: each block's two streams are
+// decoded once for all NT tiles of pairs. As do_tile otherwise (the same float
+// operations per pair); the pair scales come from memory (LDS has no room for NT
+// sets beside the tables), one step ahead with the activations.
+template <bool GU, int TY, int NT>
+__device__ __forceinline__ void do_tiles(const GroupArgs& a, const int4& tk, int tl, uint8_t* lds, uint8_t* wl, int lane,
+                                         uint32_t& sunk) {
+    const int col = lane & 15, e4 = lane >> 4, nb = (GU ? a.dim : a.ff) / 256;
+    const uint32_t mk = e4 < 2 ? ~0u : 0u;
+    Stream st[2];
+    const uint8_t* planes[2];
+    uint32_t row0nb[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        const MatRef m = mat_at(a.descs, tk.x, GU ? s : 2);
+        const int row0 = GU ? 16 * tl : 32 * tl + 16 * s;
+        row0nb[s] = uint32_t(row0 * nb);
+        st[s] = Stream{rsrc(m.base), uint32_t((row0 + col) * nb), uint32_t(m.off1), uint32_t(m.off2)};
+        planes[s] = m.base + (TY == kIQ2_XXS ? m.off1 : m.off2) + size_t(row0) * nb * 2;
+    }
+    const __amdgpu_buffer_rsrc_t rx = rsrc((GU ? a.xq : a.hq) + tile_off(tk.y >> 4, nb));
+    const __amdgpu_buffer_rsrc_t rp = rsrc((GU ? a.xd : a.hd) + size_t(tk.y >> 4) * nb * 16);
+    const uint32_t va = 256u * e4 + 16u * col;
+    struct Step {   // one block's activations and scales of one tile
+        Act<TY> x;
+        uint4 d;
+    };
+    Step p0, p1;
+    auto load_p = [&](Step& p, int blk, int mt) {
+        const uint32_t t = uint32_t(mt) * uint32_t(nb) * 5120u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p.x.a[i] = ld128(rx, va + 4096u * blk + 1024u * i, t);
+        if constexpr (TY == kIQ1_M) p.x.a[4] = ld128(rx, va + 1024u * blk, t + 4096u * nb);
+        p.d = ld128(rp, 64u * blk + 16u * e4, uint32_t(mt) * uint32_t(nb) * 64u);
+    };
+    Raw w0[2], w1[2];   // IQ2
+    uint32_t t0 = 0;
+    auto load_w = [&](Raw (&w)[2], int blk) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) load_raw<TY>(w[s], st[s], blk, e4);
+    };
+    auto touch2 = [&](int blk) { return touch(st[0], blk) ^ touch(st[1], blk); };
+    Raw1 r1[2];         // IQ1_M
+    if constexpr (TY == kIQ1_M) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) load_raw1(r1[s], st[s], row0nb[s], 0, nb, lane);
+    } else {
+        load_w(w0, 0);
+        t0 = touch2(min(3, nb - 1));
+    }
+    load_p(p0, 0, 0);
+    uint16_t* rd = reinterpret_cast<uint16_t*>(wl + 64 * kGrpNb);
+    if constexpr (TY != kIQ1_M) {
+        wave_sync();   // the previous tile's are read
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+            for (int i = lane; i < 2 * nb; i += 64)
+                reinterpret_cast<uint4*>(rd + 16 * kGrpNb * s)[i] = reinterpret_cast<const uint4*>(planes[s])[i];
+        wave_sync();
+    }
+    float acc[NT][2][4];
+#pragma unroll
+    for (int mt = 0; mt < NT; ++mt)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[mt][s][r] = 0.0f;
+    // Block b from its raw words; `odd` (with NT odd, the block's parity) says which
+    // set holds its first step.
+    auto block = [&](const Raw (&w)[2], int b, auto odd) {
+        Dec dec[2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) decode<TY>(dec[s], w[s], lds, lane, e4);
+        float d[2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) d[s] = TY == kIQ1_M ? dec[s].d : h2f(rd[16 * kGrpNb * s + col * nb + b]);
+#pragma unroll
+        for (int mt = 0; mt < NT; ++mt) {
+            Step& now = (mt + odd.value) & 1 ? p1 : p0;
+            Step& then = (mt + odd.value) & 1 ? p0 : p1;
+            load_p(then, mt + 1 < NT ? b : min(b + 1, nb - 1), mt + 1 < NT ? mt + 1 : 0);
+            __builtin_amdgcn_sched_barrier(0);   // the loads stay ahead of the compute
+            int bi[2][4];
+            if constexpr (TY == kIQ1_M) {
+#pragma unroll
+                for (int s = 0; s < 2; ++s) products1<4>(dec[s], now.x, bi[s]);
+            } else {
+                products<TY, 4>(dec, now.x, mk, bi);
+            }
+            const float xd[4] = {__uint_as_float(now.d.x), __uint_as_float(now.d.y), __uint_as_float(now.d.z), __uint_as_float(now.d.w)};
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[mt][s][r] = fmaf(__fmul_rn(d[s], xd[r]), float(bi[s][r]), acc[mt][s][r]);
+        }
+    };
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, NT & 1> second{};   // odd NT: the second block of a pair starts in p1
+    if constexpr (TY == kIQ1_M) {
+        uint8_t* raw = wl + 64 * kGrpNb;
+        for (int b = 0; b < nb; b += 4) {
+            wave_sync();   // the previous four are read
+#pragma unroll
+            for (int s = 0; s < 2; ++s) store_raw1(raw + kRaw1 * s, r1[s], lane);
+            wave_sync();
+#pragma unroll
+            for (int s = 0; s < 2; ++s) load_raw1(r1[s], st[s], row0nb[s], min(b + 4, nb - 1), nb, lane);
+            for (int i = 0; i < 4; i += 2) {
+                if (b + i >= nb) break;
+                Raw w[2];
+#pragma unroll
+                for (int s = 0; s < 2; ++s) read_raw1(w[s], raw + kRaw1 * s, i, col, e4);
+                block(w, b + i, even);
+                if (b + i + 1 >= nb) break;
+#pragma unroll
+                for (int s = 0; s < 2; ++s) read_raw1(w[s], raw + kRaw1 * s, i + 1, col, e4);
+                block(w, b + i + 1, second);
+            }
+        }
+    } else {
+        for (int b = 0; b < nb; b += 2) {
+            load_w(w1, min(b + 1, nb - 1));
+            sink(sunk, t0);
+            t0 = touch2(min(b + 5, nb - 1));
+            block(w0, b, even);
+            load_w(w0, min(b + 2, nb - 1));
+            if (b + 1 < nb) block(w1, b + 1, second);
+        }
+        sink(sunk, t0);
+    }
+#pragma unroll
+    for (int mt = 0; mt < NT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int j = 16 * mt + 4 * r + e4;   // the pair of tile position 4 e4 + r
+            if (j < tk.z) {
+                const size_t p = size_t(a.order[tk.y + j]);
+                if constexpr (GU) {
+                    a.h[p * a.ff + 16 * tl + col] =
+                        silu_mul3(__fmul_rn(0.125f, acc[mt][0][r]), __fmul_rn(0.125f, acc[mt][1][r]), a.lim);
+                } else {
+                    float* y = a.y + p * a.dim + 32 * tl + col;
+                    y[0] = __fmul_rn(0.125f, acc[mt][0][r]);
+                    y[16] = __fmul_rn(0.125f, acc[mt][1][r]);
+                }
+            }
+        }
+}
+
 // MASK: block types among the launch's matrices (bits 1 IQ2_XXS, 2 IQ2_XS, 4 IQ1_M).
-template <bool GU, int MASK, int NW, bool TR>
+// MT: tasks may hold up to 16 MT pairs.
+template <bool GU, int MASK, int NW, int MT, bool TR>
 __global__ __launch_bounds__(NW * 64, 1) void grouped_kernel(GroupArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[grp_lds_bytes(MASK, NW)];
     __shared__ uint32_t s_bundle;   // current bundle << 8 | its next tile
@@ -894,9 +1051,19 @@ __global__ __launch_bounds__(NW * 64, 1) void grouped_kernel(GroupArgs a) {
             if (tile >= total) break;
             const int task = tile / tiles, tl = tile - task * tiles;
             const int4 tk = task_at((GU ? a.tasks : a.dtasks) + base, task);
-            if (MASK == 1 || (MASK == 7 && ti == 0)) do_tile<GU, kIQ2_XXS, TR, NW <= 8>(a, tk, tl, lds, wl, lane, sunk);
-            else if (MASK == 2 || (MASK == 7 && ti == 1)) do_tile<GU, kIQ2_XS, TR, NW <= 8>(a, tk, tl, lds, wl, lane, sunk);
-            else do_tile<GU, kIQ1_M, TR, NW <= 8>(a, tk, tl, lds, wl, lane, sunk);
+            const auto tile_of = [&]<int TY>() {
+                if constexpr (MT == 1) {
+                    do_tile<GU, TY, TR, NW <= 8>(a, tk, tl, lds, wl, lane, sunk);
+                } else {
+                    if (tk.z <= 16) do_tiles<GU, TY, 1>(a, tk, tl, lds, wl, lane, sunk);
+                    else if (tk.z <= 32) do_tiles<GU, TY, 2>(a, tk, tl, lds, wl, lane, sunk);
+                    else if (tk.z <= 48) do_tiles<GU, TY, 3>(a, tk, tl, lds, wl, lane, sunk);
+                    else do_tiles<GU, TY, 4>(a, tk, tl, lds, wl, lane, sunk);
+                }
+            };
+            if (MASK == 1 || (MASK == 7 && ti == 0)) tile_of.template operator()<kIQ2_XXS>();
+            else if (MASK == 2 || (MASK == 7 && ti == 1)) tile_of.template operator()<kIQ2_XS>();
+            else tile_of.template operator()<kIQ1_M>();
         }
     }
     if (sunk == 0x9e3779b9u && lane == 64) (GU ? a.h : a.y)[0] = 0.0f;   // never true (lane < 64): keeps the touches
@@ -963,10 +1130,14 @@ hipError_t launch_grouped(GroupArgs args, int gu_types, int dn_types, int cus, h
     // 50 registers at 3 (512 tokens, 4096 x 3072, 384 experts: 1,426 against 1,494 us)
     constexpr int NW = 12, NWM = 8;
     if (args.T < 1 || args.k < 1 || args.k > 16 || args.n_experts > kGroupMaxExperts || args.dim % 256 || args.ff % 256 ||
-        args.dim > kGrpNb * 256 || args.ff > 4096 || args.cap < kTile || args.cap % kTile)
+        args.dim > kGrpNb * 256 || args.ff > 4096)
         return hipErrorNotSupported;
     const bool trace = args.tq8x || args.tq8h || args.th || args.tint;
     if (trace && (gu_types != 1 || dn_types != 2)) return hipErrorNotSupported;
+    const int64_t pairs = int64_t(args.T) * args.k, experts = pairs < args.n_experts ? pairs : args.n_experts;
+    const bool multi = !trace && (pairs >= int64_t(kMultiPairs) * args.n_experts ||
+                                  experts * std::max(args.ff / 16, args.dim / 32) <= 8 * int64_t(cus));
+    args.cap = multi ? 64 : 16;
     const int P = args.T * args.k, nbx = args.dim / 256, nbh = args.ff / 256;
     const auto grouped = [&](auto kernel, int nw = 12) { hipLaunchKernelGGL(kernel, dim3(cus), dim3(nw * 64), 0, s, args); };
     const auto rows = [&](auto kernel, const float* src, int n, int nb, int8_t* q, float* d, uint8_t* tr) {
@@ -978,20 +1149,36 @@ hipError_t launch_grouped(GroupArgs args, int gu_types, int dn_types, int cus, h
     hipLaunchKernelGGL(bucket_kernel, dim3(1), dim3(1024), 0, s, args);
     if (trace) {   // the parity trace (separate instances)
         rows((q8k_rows_kernel<ROWS_X, false, true>), args.x, args.T, nbx, args.xq, args.xd, args.tq8x);
-        grouped(grouped_kernel<true, 1, NW, true>);
+        grouped(grouped_kernel<true, 1, NW, 1, true>);
         rows((q8k_rows_kernel<ROWS_H, false, true>), args.h, P, nbh, args.hq, args.hd, args.tq8h);
-        grouped(grouped_kernel<false, 2, NW, true>);
+        grouped(grouped_kernel<false, 2, NW, 1, true>);
     } else {
         rows(gu_types & 4 ? q8k_rows_kernel<ROWS_X, true, false> : q8k_rows_kernel<ROWS_X, false, false>, args.x, args.T, nbx,
              args.xq, args.xd, nullptr);
-        if (gu_types == 1) grouped(grouped_kernel<true, 1, NW, false>);
-        else if (gu_types == 4) grouped(grouped_kernel<true, 4, NW, false>);
-        else grouped(grouped_kernel<true, 7, NWM, false>, NWM);
+        if (multi) {
+            if (gu_types == 1) grouped(grouped_kernel<true, 1, 8, 4, false>, 8);
+            else if (gu_types == 4) grouped(grouped_kernel<true, 4, 8, 4, false>, 8);
+            else grouped(grouped_kernel<true, 7, 8, 4, false>, 8);
+        } else if (gu_types == 1) {
+            grouped(grouped_kernel<true, 1, NW, 1, false>);
+        } else if (gu_types == 4) {
+            grouped(grouped_kernel<true, 4, NW, 1, false>);
+        } else {
+            grouped(grouped_kernel<true, 7, NWM, 1, false>, NWM);
+        }
         rows(dn_types & 4 ? q8k_rows_kernel<ROWS_H, true, false> : q8k_rows_kernel<ROWS_H, false, false>, args.h, P, nbh,
              args.hq, args.hd, nullptr);
-        if (dn_types == 2) grouped(grouped_kernel<false, 2, NW, false>);
-        else if (dn_types == 4) grouped(grouped_kernel<false, 4, NW, false>);
-        else grouped(grouped_kernel<false, 7, NWM, false>, NWM);
+        if (multi) {
+            if (dn_types == 2) grouped(grouped_kernel<false, 2, 8, 4, false>, 8);
+            else if (dn_types == 4) grouped(grouped_kernel<false, 4, 8, 4, false>, 8);
+            else grouped(grouped_kernel<false, 7, 8, 4, false>, 8);
+        } else if (dn_types == 2) {
+            grouped(grouped_kernel<false, 2, NW, 1, false>);
+        } else if (dn_types == 4) {
+            grouped(grouped_kernel<false, 4, NW, 1, false>);
+        } else {
+            grouped(grouped_kernel<false, 7, NWM, 1, false>, NWM);
+        }
     }
     const bool al16 = (reinterpret_cast<uintptr_t>(args.out) | reinterpret_cast<uintptr_t>(args.shared)) % 16 == 0;
     if (al16) hipLaunchKernelGGL(gcombine_kernel<4>, dim3((args.dim / 4 + 255) / 256, args.T), dim3(256), 0, s, args);

@@ -136,8 +136,8 @@ struct GroupArgs {
     int32_t* pos;               // slot of each pair (P; -1 for a bad id), with order bits (xl_grouped.hip)
     int4* tasks; int4* dtasks;  // (expert, first slot, pairs, 0) per task, by gate type and by down type
     GroupQueue* queue;          // task counts and work queues, written by the bucket kernel
-    int cap;
-    int gu_first, dn_first;     // the queues' first bundles (set by launch_grouped)
+    int cap;                    // set by launch_grouped, as
+    int gu_first, dn_first;     // the queues' first bundles
     float* h;                   // P * ff
     int8_t* hq; float* hd;      // Q8_K(h): as xq and xd, of ff
     float* y;                   // P * dim

@@ -63,3 +63,30 @@ def test_grouped_types(orc, kind, dim, ff, E, T, k, skew, lim):
             rows.append(orc.expert(tt, *orc.gen_expert(tt, 21, 0, int(e), dim, ff), dim, ff, x[t], limit=lim))
         want = orc.combine(ids[t], w[t], np.stack(rows), shared[t])
         assert max_rel(got[t], want) < TOL, (t, max_rel(got[t], want))
+
+
+@pytest.mark.parametrize("dim,ff", [(1024, 512), (768, 256), (2304, 1024)])
+def test_tasks_of_several_tiles(dim, ff):
+    """Many pairs per expert: tasks of up to 64 pairs (1 to 4 tiles and their
+    remainders) give the bits of 16-pair tasks, which the traced call keeps."""
+    counts = [16, 17, 32, 33, 48, 49, 64, 65, 1, 129, 15]
+    print(f"[gpu-step] tasks of several tiles {dim}x{ff}", flush=True)
+    E, T = len(counts), sum(counts)
+    rng = np.random.default_rng(dim)
+    ids = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int32).reshape(T, 1)
+    types = np.zeros((1, E, 3), np.int32)
+    types[..., :2], types[..., 2] = 16, 17
+    d_ids = torch.from_numpy(ids).cuda()
+    d_w = torch.from_numpy(rng.random((T, 1)).astype(np.float32)).cuda()
+    d_x = torch.from_numpy(rng.standard_normal((T, dim)).astype(np.float32)).cuda()
+    out, traced = (torch.zeros((T, dim), dtype=torch.float32, device="cuda") for _ in range(2))
+    y = torch.zeros((T, dim), dtype=torch.float32, device="cuda")
+    q8x = torch.zeros(T * (dim // 256) * 292, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    with xl.Lane(dim, ff, 1, E, types, max_picks=1, max_tokens=T) as lane:
+        lane.generate(seed=4)
+        lane.grouped_forward_async(0, d_ids, d_w, d_x, out)
+        lane.grouped_trace_async(0, d_ids, d_w, d_x, traced, q8x=q8x, y=y)
+        lane.sync()
+    assert float(out.abs().max()) > 0
+    assert torch.equal(out.view(torch.int32), traced.view(torch.int32))
