@@ -567,22 +567,19 @@ SharedWork shared_work(int dim, int ff, int T) {
 }
 
 // Enqueues the per32 layer (hip_resident_bank.hpp:185-200 with the kernels of
-// hip_experts.hip): quant32(x), gate and up rows of every pick in one launch,
-// SwiGLU, quant32(h) of every pick, down rows into y (k x dim), then the
+// hip_experts.hip): quant32(x) with the gate and up rows of every pick in one
+// launch, SwiGLU, quant32(h) of every pick, down rows into y (k x dim) with the
 // fixed-order combine into out when out is given.
 void enqueue_per32(xl_context* ctx, int32_t layer, const int32_t* d_ids, const float* d_w, int32_t k, const float* d_x,
                    const float* d_shared, float* d_y, float* d_out, hipStream_t s) {
     const int dim = ctx->cfg.dim, ff = ctx->cfg.ff, E = ctx->cfg.n_experts;
     const xl::ExpertDesc* descs = ctx->d_descs + size_t(layer) * E;
-    float* xd = ctx->p32d;
     float* hd = ctx->p32d + ctx->act_max / 32;
     const xl::MatRef none{};
     Marks mark(ctx, s);
     mark("");
-    hip_check(xl::dev::launch_quant32(d_x, 1, dim, ctx->xq, xd, ctx->err_flag, s), "quant32(x) launch");
-    mark("quant32_x");
-    hip_check(xl::dev::launch_mv32(descs, d_ids, none, none, k, E, 0, 2, ff, dim, ctx->xq, 0, xd, 0, ctx->g, ctx->u,
-                                   size_t(ff), ctx->tables, ctx->err_flag, s),
+    hip_check(xl::dev::launch_gate_up32(descs, d_ids, k, E, ctx->gu_mask[size_t(layer)], ff, dim, d_x, ctx->g, ctx->u,
+                                        ctx->tables, ctx->cus, ctx->err_flag, s),
               "per32 gate/up launch");
     mark("gate_up32");
     hip_check(xl::dev::launch_swiglu_quant32(ctx->g, ctx->u, k, ff, ctx->cfg.swiglu_limit, ctx->hq, hd, s),
@@ -591,10 +588,15 @@ void enqueue_per32(xl_context* ctx, int32_t layer, const int32_t* d_ids, const f
     // the fixed-order combine (runtime.cpp:183-188) in the down launch's epilogue
     // when out is given: each workgroup holds every pick's value of its rows
     const xl::dev::Mv32Comb cb{d_w, d_shared, d_out};
-    hip_check(xl::dev::launch_mv32(descs, d_ids, none, none, k, E, 2, 1, dim, ff, ctx->hq, size_t(ff), hd, size_t(ff / 32),
-                                   d_y, nullptr, size_t(dim), ctx->tables, ctx->err_flag, s, nullptr,
-                                   d_out ? &cb : nullptr),
-              "per32 down launch");
+    const hipError_t e = xl::dev::launch_down32(descs, d_ids, k, E, ctx->dn_mask[size_t(layer)], dim, ff, ctx->hq, hd, d_y, cb,
+                                              ctx->tables, ctx->cus, ctx->err_flag, s);
+    if (e == hipErrorNotSupported)   // its hidden rows or its workgroup's outputs do not fit LDS
+        hip_check(xl::dev::launch_mv32(descs, d_ids, none, none, k, E, 2, 1, dim, ff, ctx->hq, size_t(ff), hd, size_t(ff / 32),
+                                       d_y, nullptr, size_t(dim), ctx->tables, ctx->err_flag, s, nullptr,
+                                       d_out ? &cb : nullptr),
+                  "per32 down launch");
+    else
+        hip_check(e, "per32 down launch");
     mark(d_out ? "down32_combine" : "down32");
 }
 

@@ -257,6 +257,16 @@ hipError_t launch_mv32(const ExpertDesc* descs, const int32_t* ids, const MatRef
                        const float* d, size_t d_stride, float* y0, float* y1, size_t y_stride,
                        const uint64_t* tables, int* err, hipStream_t s, const Mv32Post* epi = nullptr,
                        const Mv32Comb* comb = nullptr);
+// The bank rows of the per32 layer (xl_per32_rows.hip) with launch_mv32's bits:
+// gate/up of every pick with x quantized in the launch, and down with its
+// combine (cb.out null: y alone). mask: the block types among the layer's
+// matrices of these roles. hipErrorNotSupported (down): more than its LDS holds.
+hipError_t launch_gate_up32(const ExpertDesc* descs, const int32_t* ids, int picks, int n_experts, int mask, int n,
+                            int k, const float* x, float* g, float* u, const uint64_t* tables, int cus, int* err,
+                            hipStream_t s);
+hipError_t launch_down32(const ExpertDesc* descs, const int32_t* ids, int picks, int n_experts, int mask, int n, int k,
+                         const int8_t* q, const float* d, float* y, const Mv32Comb& cb, const uint64_t* tables, int cus,
+                         int* err, hipStream_t s);
 // Hyper-connection post (sycl/hc/core.hpp:81-86) of T tokens, H <= 4 streams
 // of D: out[t][k][e] = post[t][k] * y[t][e] + sum_j comb[t][j * H + k] *
 // res[t][j][e]; out may equal res (in place).
