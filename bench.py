@@ -499,7 +499,7 @@ def main():
               1: "xl::dev::stream_kernel (single-launch layer, IQ2 instance)",
               2: "xl::dev::stream_kernel (single-launch layer, IQ1_M instance)",
               3: "xl::dev::stream_kernel (single-launch layer, mixed-type instance)",
-              4: "grouped path (bucket, Q8_K, gu_kernel, Q8_K, dn_kernel, combine: 6 launches per step)"}.get(cfg)
+              4: "grouped path (bucket, Q8_K, grouped_kernel gate/up, Q8_K, grouped_kernel down, combine: 6 launches per step)"}.get(cfg)
     if cfg == 6:   # whichever single launch served the calls (xl_debug_launch_counts)
         counts = lane.launch_counts()
         kernel = ("xl::dev::stream_kernel (single-launch layer, IQ2 instance, 5120 x 2304)" if counts["stream"]
@@ -510,8 +510,8 @@ def main():
                   "prologue), mv32 shared gate+up, swiglu_quant32, mv32 shared down (+ the routed row, hc_post in "
                   "its epilogue): 4 launches per step")
     if args.per32:
-        kernel = ("per32 chain (quant32, mv32 gate+up, swiglu_quant32, mv32 down with the fixed-order combine in its "
-                  "epilogue: 4 launches per step)")
+        kernel = ("per32 chain (rows32 gate+up with x quantized in it, swiglu_quant32, rows32 down with the fixed-order "
+                  "combine: 3 launches per step)")
     traffic = measured_traffic() if cfg == 1 and not args.per32 else None
 
     cpu = None

@@ -1,5 +1,5 @@
 // CDNA4 (gfx950) grouped routed-expert path: T tokens, each with its own k
-// picks, reading every touched expert's weights once per 16 of its (token,
+// picks, reading every touched expert's weights once per task of its (token,
 // pick) pairs. The result is that of T independent layer calls
 // (WarmRedirect::warm_compute_many per token, engine/strata/warm/runtime.hpp:13,
 // then the fixed-order join of runtime.cpp:183-188): per (row, pair) the same
@@ -7,7 +7,7 @@
 // block order as the row kernels.
 //
 //   bucket_kernel    one workgroup: pairs bucketed by expert id into tasks of
-//                    at most 16 pairs of one expert
+//                    at most 16 or 64 pairs of one expert
 //   q8k_rows_kernel  Q8_K (q8k_core.hpp:30-38) of token rows (x) and pair rows
 //                    (h), written in the operand order of the MFMA kernels
 //   grouped_kernel   gate/up + SwiGLU of every task, then down of every task

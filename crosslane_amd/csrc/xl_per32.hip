@@ -17,6 +17,7 @@
 //                   clamped first when the SwiGLU limit is set), quantized per
 //                   32 as quant32_kernel does
 //
+// The layer's rows over the bank have kernels of their own (xl_per32_rows.hip).
 // The bank's planar blocks are decoded directly (xl_format.hpp layout); the
 // codebooks come from the context's expanded tables. The dense formats of the
 // shared-expert matrices (Q8_0, Q4_K, Q5_K, Q6_K) are read as raw ggml blocks:

@@ -167,7 +167,7 @@ int32_t xl_sync(xl_context* ctx, void* stream, xl_error* err);
  * shared and out T x dim. The result is that of T xl_layer_forward calls (per
  * token: WarmRedirect::warm_compute_many, engine/strata/warm/runtime.hpp:13,
  * then warm_execute's fixed-order combine, runtime.cpp:180-188), with every
- * touched expert's weights read once per 16 of its (token, pick) pairs on
+ * touched expert's weights read once per task of its (token, pick) pairs on
  * int8 MFMA: IQ2_XXS gate/up + IQ2_XS down layers always, layers of other or
  * mixed types from 13 tokens on (below, one layer call per token). Needs a context opened with max_tokens >= T; picks
  * of one token unique. The async form takes device pointers and checks ids on
