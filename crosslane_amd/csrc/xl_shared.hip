@@ -367,7 +367,7 @@ __global__ __launch_bounds__(256) void quant32t_kernel(const float* __restrict__
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[j] = p[j];
     }
-    float am = 0.0f;
+    float am = fabsf(v[0]);   // no start value: a block of NaNs keeps NaN, as in quant32_kernel
     bool finite = true;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -443,7 +443,8 @@ __global__ __launch_bounds__(SPLIT ? 1024 : 512, 4) void ffn_gu_kernel(const uin
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 g[rt][tt][r] = silu_mul3(g[rt][tt][r], u[rt][tt][r], lim);
-                am = fmaxf(am, fabsf(g[rt][tt][r]));
+                // the first value starts the maximum: a block of NaNs keeps NaN, as in swiglu_quant32_kernel
+                am = rt + r == 0 ? fabsf(g[rt][tt][r]) : fmaxf(am, fabsf(g[rt][tt][r]));
             }
         am = fmaxf(am, __shfl_xor(am, 16));
         am = fmaxf(am, __shfl_xor(am, 32));

@@ -50,3 +50,28 @@ def test_tokens_equal_single_calls(types, dim, ff, T, lim):
             want = one.cpu().numpy().view(np.uint32)
             assert np.array_equal(outs[0][t].view(np.uint32), want), t
             assert np.array_equal(outs[1][t].view(np.uint32), want), t
+
+
+@pytest.mark.parametrize("T", [3, 16, 33, 512])
+def test_a_sub_block_of_nans_stays_nan(T):
+    """32 gate rows whose scales are NaN make one per-32 block of h NaN in all its
+    values, and with it the block's scale and every output, as in a single call; NaNs
+    beside finite values of h take no part in the block's maximum."""
+    print(f"[gpu-step] shared FFN, NaN rows, T={T}", flush=True)
+    dim, ff = 256, 2048
+    for rows in (32, 31):                # the whole block; one finite value in it
+        mats = [dense_matrix(8, *((ff, dim) if r < 2 else (dim, ff)), seed=r).copy() for r in range(3)]
+        mats[0].reshape(ff, dim // 32, 34)[64:64 + rows, :, :2] = np.frombuffer(np.float16("nan").tobytes(), np.uint8)
+        mats = [dev(m) for m in mats]
+        dx = dev(np.random.default_rng(T).standard_normal((T, dim)).astype(np.float32))
+        work = torch.empty(xl.shared_work_bytes(dim, ff, T), dtype=torch.uint8, device="cuda")
+        out, one = torch.zeros((T, dim), device="cuda"), torch.zeros(dim, device="cuda")
+        torch.cuda.synchronize()
+        with xl.Lane(dim, 256, 1, 1, np.full((1, 1, 3), 29, np.int32)) as lane:
+            lane.shared_forward_async((8, 8, 8), *mats, ff, dx, out, work)
+            for t in (0, T - 1):
+                lane.shared_forward_async((8, 8, 8), *mats, ff, dx[t], one, work)
+                lane.sync()
+                assert bool(torch.isnan(one).all()) == (rows == 32)
+                assert int((torch.isnan(out[t]) != torch.isnan(one)).sum()) == 0, (rows, t)
+                assert rows == 32 or int((out[t].view(torch.int32) != one.view(torch.int32)).sum()) == 0, (rows, t)
