@@ -234,6 +234,9 @@ __device__ __forceinline__ void tile_rows(const uint8_t* W, int nb, const ActTil
                                                               16 * act[tt].t);
             xd[tt] = *reinterpret_cast<const float4*>(act[tt].d + size_t(bc * act[tt].nt + act[tt].t) * 8 + 4 * par);
         }
+        // This wave's copies of step s have arrived, stated here: nothing in the language
+        // ties a copy to LDS to the barrier that hands it to the other waves.
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
         __syncthreads();   // step s is in LDS, and every wave is done with step s - 1
         if (s + 1 < steps) stage_step<TY>(lds + ((s + 1) & 1) * kStepBytes<TY>, W, row_bytes, nb, s + 1, w, lane);
         if (b >= nb) continue;   // wave-uniform; the step's barriers are the loop's
