@@ -638,8 +638,28 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
 }
+// The float sum of a row, over its blocks in order: one fma chain, or (F8) a chain
+// per eight blocks, the chains' results added up in order. Layers of other types
+// than IQ2_XXS gate/up with IQ2_XS down take F8: with fewer than kGroupAnyTokens
+// tokens they are layer calls, whose sums are trees, and one chain over 12 to 20
+// blocks is further from 64 bits than those. Tokens without a moved quant of h,
+// IQ1_M, from 64 bits: 4096 x 3072 one chain 1.44e-7, layer calls 1.32e-7, by eights
+// 1.26e-7; 5120 x 2304 1.47e-7, 1.33e-7, 1.27e-7; mixed types 1.38e-7, 1.26e-7,
+// 1.20e-7. By fours 1.24e-7, but the several-tile kernels then spill (IQ1_M, 2,048
+// tokens of 64 experts: 2,053 us; by eights 1,427; one chain 1,418).
+// Before block b > 0, and past the row's last block with b = 0:
+template <bool F8, int N>
+__device__ __forceinline__ void next_chain(float* acc, float* total, int b, int nb) {
+    if (!F8 || (b & 7) || (b == 0 && nb <= 8)) return;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float v = b == 8 ? acc[i] : __fadd_rn(total[i], acc[i]);
+        total[i] = v;
+        acc[i] = b == 0 ? v : 0.0f;
+    }
+}
 // TR: also write each pair's block integers (GroupArgs::tint).
-template <bool GU, int TY, bool TR, bool DB>
+template <bool GU, int TY, bool TR, bool DB, bool F8>
 __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int tl, uint8_t* lds, uint8_t* wl, int lane,
                                         uint32_t& sunk) {
     const int col = lane & 15, e4 = lane >> 4, nb = (GU ? a.dim : a.ff) / 256;
@@ -711,7 +731,7 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
     wave_sync();
     // RR: output registers that can hold a pair (ceil(pairs / 4), rounded up to 2 or 4)
     auto run = [&]<int RR>() {
-        float acc[2][4] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+        float acc[2][4] = {}, total[2][4];
         int blk_c = 0;   // block the next compute() handles
         auto compute = [&](const Raw (&w)[2], const Act<TY>& x) {
             const int b = blk_c++;
@@ -752,6 +772,7 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
             // meanwhile
             uint8_t* raw = wl + 64 * kGrpNb;
             for (int b = 0; b < nb; b += 4) {
+                if (b > 0) next_chain<F8, 8>(acc[0], total[0], b, nb);
                 wave_sync();   // the previous four are read
 #pragma unroll
                 for (int s = 0; s < 2; ++s) store_raw1(raw + kRaw1 * s, r1[s], lane);
@@ -778,6 +799,7 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
             // so no wait ever covers a load issued in the same step); line touches four
             // blocks ahead in fixed registers, one per line of two blocks.
             for (int b = 0; b < nb; b += 4) {
+                if (b > 0) next_chain<F8, 8>(acc[0], total[0], b, nb);
                 load(w1, x1, min(b + 1, nb - 1));
                 sink(sunk, t0);
                 t0 = touch2(min(b + 5, nb - 1));
@@ -797,6 +819,7 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
             }
             sink(sunk, t0 ^ t2);
         }
+        next_chain<F8, 8>(acc[0], total[0], 0, nb);
 #pragma unroll
         for (int r = 0; r < RR; ++r)
             if (po[r] >= 0) {
@@ -818,7 +841,7 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
 // decoded once for all NT tiles of pairs. As do_tile otherwise (the same float
 // operations per pair); the pair scales come from memory (LDS has no room for NT
 // sets beside the tables), one step ahead with the activations.
-template <bool GU, int TY, int NT>
+template <bool GU, int TY, int NT, bool F8>
 __device__ __forceinline__ void do_tiles(const GroupArgs& a, const int4& tk, int tl, uint8_t* lds, uint8_t* wl, int lane,
                                          uint32_t& sunk) {
     const int col = lane & 15, e4 = lane >> 4, nb = (GU ? a.dim : a.ff) / 256;
@@ -874,13 +897,7 @@ __device__ __forceinline__ void do_tiles(const GroupArgs& a, const int4& tk, int
                 reinterpret_cast<uint4*>(rd + 16 * kGrpNb * s)[i] = reinterpret_cast<const uint4*>(planes[s])[i];
         wave_sync();
     }
-    float acc[NT][2][4];
-#pragma unroll
-    for (int mt = 0; mt < NT; ++mt)
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[mt][s][r] = 0.0f;
+    float acc[NT][2][4] = {}, total[NT][2][4];
     // Block b from its raw words; `odd` (with NT odd, the block's parity) says which
     // set holds its first step.
     auto block = [&](const Raw (&w)[2], int b, auto odd) {
@@ -915,6 +932,7 @@ __device__ __forceinline__ void do_tiles(const GroupArgs& a, const int4& tk, int
     if constexpr (TY == kIQ1_M) {
         uint8_t* raw = wl + 64 * kGrpNb;
         for (int b = 0; b < nb; b += 4) {
+            if (b > 0) next_chain<F8, 8 * NT>(acc[0][0], total[0][0], b, nb);
             wave_sync();   // the previous four are read
 #pragma unroll
             for (int s = 0; s < 2; ++s) store_raw1(raw + kRaw1 * s, r1[s], lane);
@@ -935,6 +953,7 @@ __device__ __forceinline__ void do_tiles(const GroupArgs& a, const int4& tk, int
         }
     } else {
         for (int b = 0; b < nb; b += 2) {
+            if (b > 0) next_chain<F8, 8 * NT>(acc[0][0], total[0][0], b, nb);
             load_w(w1, min(b + 1, nb - 1));
             sink(sunk, t0);
             t0 = touch2(min(b + 5, nb - 1));
@@ -944,6 +963,7 @@ __device__ __forceinline__ void do_tiles(const GroupArgs& a, const int4& tk, int
         }
         sink(sunk, t0);
     }
+    next_chain<F8, 8 * NT>(acc[0][0], total[0][0], 0, nb);
 #pragma unroll
     for (int mt = 0; mt < NT; ++mt)
 #pragma unroll
@@ -965,7 +985,8 @@ __device__ __forceinline__ void do_tiles(const GroupArgs& a, const int4& tk, int
 
 // MASK: block types among the launch's matrices (bits 1 IQ2_XXS, 2 IQ2_XS, 4 IQ1_M).
 // MT: tasks may hold up to 16 MT pairs.
-template <bool GU, int MASK, int NW, int MT, bool TR>
+// F8: the order of the float sums (do_tile).
+template <bool GU, int MASK, int NW, int MT, bool TR, bool F8>
 __global__ __launch_bounds__(NW * 64, 1) void grouped_kernel(GroupArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[grp_lds_bytes(MASK, NW)];
     __shared__ uint32_t s_bundle;   // current bundle << 8 | its next tile
@@ -1053,12 +1074,12 @@ __global__ __launch_bounds__(NW * 64, 1) void grouped_kernel(GroupArgs a) {
             const int4 tk = task_at((GU ? a.tasks : a.dtasks) + base, task);
             const auto tile_of = [&]<int TY>() {
                 if constexpr (MT == 1) {
-                    do_tile<GU, TY, TR, NW <= 8>(a, tk, tl, lds, wl, lane, sunk);
+                    do_tile<GU, TY, TR, NW <= 8, F8>(a, tk, tl, lds, wl, lane, sunk);
                 } else {
-                    if (tk.z <= 16) do_tiles<GU, TY, 1>(a, tk, tl, lds, wl, lane, sunk);
-                    else if (tk.z <= 32) do_tiles<GU, TY, 2>(a, tk, tl, lds, wl, lane, sunk);
-                    else if (tk.z <= 48) do_tiles<GU, TY, 3>(a, tk, tl, lds, wl, lane, sunk);
-                    else do_tiles<GU, TY, 4>(a, tk, tl, lds, wl, lane, sunk);
+                    if (tk.z <= 16) do_tiles<GU, TY, 1, F8>(a, tk, tl, lds, wl, lane, sunk);
+                    else if (tk.z <= 32) do_tiles<GU, TY, 2, F8>(a, tk, tl, lds, wl, lane, sunk);
+                    else if (tk.z <= 48) do_tiles<GU, TY, 3, F8>(a, tk, tl, lds, wl, lane, sunk);
+                    else do_tiles<GU, TY, 4, F8>(a, tk, tl, lds, wl, lane, sunk);
                 }
             };
             if (MASK == 1 || (MASK == 7 && ti == 0)) tile_of.template operator()<kIQ2_XXS>();
@@ -1132,8 +1153,8 @@ hipError_t launch_grouped(GroupArgs args, int gu_types, int dn_types, int cus, h
     if (args.T < 1 || args.k < 1 || args.k > 16 || args.n_experts > kGroupMaxExperts || args.dim % 256 || args.ff % 256 ||
         args.dim > kGrpNb * 256 || args.ff > 4096)
         return hipErrorNotSupported;
-    const bool trace = args.tq8x || args.tq8h || args.th || args.tint;
-    if (trace && (gu_types != 1 || dn_types != 2)) return hipErrorNotSupported;
+    const bool trace = args.tq8x || args.tq8h || args.th || args.tint, iq2 = gu_types == 1 && dn_types == 2;
+    if (trace && !iq2) return hipErrorNotSupported;
     const int64_t pairs = int64_t(args.T) * args.k, experts = pairs < args.n_experts ? pairs : args.n_experts;
     const bool multi = !trace && (pairs >= int64_t(kMultiPairs) * args.n_experts ||
                                   experts * std::max(args.ff / 16, args.dim / 32) <= 8 * int64_t(cus));
@@ -1149,35 +1170,41 @@ hipError_t launch_grouped(GroupArgs args, int gu_types, int dn_types, int cus, h
     hipLaunchKernelGGL(bucket_kernel, dim3(1), dim3(1024), 0, s, args);
     if (trace) {   // the parity trace (separate instances)
         rows((q8k_rows_kernel<ROWS_X, false, true>), args.x, args.T, nbx, args.xq, args.xd, args.tq8x);
-        grouped(grouped_kernel<true, 1, NW, 1, true>);
+        grouped(grouped_kernel<true, 1, NW, 1, true, false>);
         rows((q8k_rows_kernel<ROWS_H, false, true>), args.h, P, nbh, args.hq, args.hd, args.tq8h);
-        grouped(grouped_kernel<false, 2, NW, 1, true>);
+        grouped(grouped_kernel<false, 2, NW, 1, true, false>);
     } else {
         rows(gu_types & 4 ? q8k_rows_kernel<ROWS_X, true, false> : q8k_rows_kernel<ROWS_X, false, false>, args.x, args.T, nbx,
              args.xq, args.xd, nullptr);
         if (multi) {
-            if (gu_types == 1) grouped(grouped_kernel<true, 1, 8, 4, false>, 8);
-            else if (gu_types == 4) grouped(grouped_kernel<true, 4, 8, 4, false>, 8);
-            else grouped(grouped_kernel<true, 7, 8, 4, false>, 8);
+            if (iq2) grouped(grouped_kernel<true, 1, 8, 4, false, false>, 8);
+            else if (gu_types == 1) grouped(grouped_kernel<true, 1, 8, 4, false, true>, 8);
+            else if (gu_types == 4) grouped(grouped_kernel<true, 4, 8, 4, false, true>, 8);
+            else grouped(grouped_kernel<true, 7, 8, 4, false, true>, 8);
+        } else if (iq2) {
+            grouped(grouped_kernel<true, 1, NW, 1, false, false>);
         } else if (gu_types == 1) {
-            grouped(grouped_kernel<true, 1, NW, 1, false>);
+            grouped(grouped_kernel<true, 1, NW, 1, false, true>);
         } else if (gu_types == 4) {
-            grouped(grouped_kernel<true, 4, NW, 1, false>);
+            grouped(grouped_kernel<true, 4, NW, 1, false, true>);
         } else {
-            grouped(grouped_kernel<true, 7, NWM, 1, false>, NWM);
+            grouped(grouped_kernel<true, 7, NWM, 1, false, true>, NWM);
         }
         rows(dn_types & 4 ? q8k_rows_kernel<ROWS_H, true, false> : q8k_rows_kernel<ROWS_H, false, false>, args.h, P, nbh,
              args.hq, args.hd, nullptr);
         if (multi) {
-            if (dn_types == 2) grouped(grouped_kernel<false, 2, 8, 4, false>, 8);
-            else if (dn_types == 4) grouped(grouped_kernel<false, 4, 8, 4, false>, 8);
-            else grouped(grouped_kernel<false, 7, 8, 4, false>, 8);
+            if (iq2) grouped(grouped_kernel<false, 2, 8, 4, false, false>, 8);
+            else if (dn_types == 2) grouped(grouped_kernel<false, 2, 8, 4, false, true>, 8);
+            else if (dn_types == 4) grouped(grouped_kernel<false, 4, 8, 4, false, true>, 8);
+            else grouped(grouped_kernel<false, 7, 8, 4, false, true>, 8);
+        } else if (iq2) {
+            grouped(grouped_kernel<false, 2, NW, 1, false, false>);
         } else if (dn_types == 2) {
-            grouped(grouped_kernel<false, 2, NW, 1, false>);
+            grouped(grouped_kernel<false, 2, NW, 1, false, true>);
         } else if (dn_types == 4) {
-            grouped(grouped_kernel<false, 4, NW, 1, false>);
+            grouped(grouped_kernel<false, 4, NW, 1, false, true>);
         } else {
-            grouped(grouped_kernel<false, 7, NWM, 1, false>, NWM);
+            grouped(grouped_kernel<false, 7, NWM, 1, false, true>, NWM);
         }
     }
     const bool al16 = (reinterpret_cast<uintptr_t>(args.out) | reinterpret_cast<uintptr_t>(args.shared)) % 16 == 0;

@@ -157,7 +157,8 @@ struct GroupArgs {
 // Measured at 4096 x 3072, 384 experts, 6 picks: 13 tokens 327 us (mixed types) and
 // 265 us (IQ1_M) grouped against 354 and 298 us by layer calls, about level at 12
 // (fewer experts or smaller shapes gain earlier: 13 tokens at 1024 x 512 take 41 us
-// against 158). Below it a call keeps the bits of its tokens' single layer calls.
+// against 158). Below it a call keeps the bits of its tokens' single layer calls; from it
+// on the float sums have another order, no further from 64 bits (next_chain).
 constexpr int kGroupAnyTokens = 13;
 constexpr int kGroupMaxExperts = 8192;
 constexpr int kRouteMaxExperts = 4096;   // router: scores and keys of one token in LDS   // experts per layer the bucket kernel counts in LDS

@@ -166,10 +166,13 @@ int32_t xl_sync(xl_context* ctx, void* stream, xl_error* err);
  * T tokens, each with its own k picks: ids and w are T x k (token-major), x,
  * shared and out T x dim. The result is that of T xl_layer_forward calls (per
  * token: WarmRedirect::warm_compute_many, engine/strata/warm/runtime.hpp:13,
- * then warm_execute's fixed-order combine, runtime.cpp:180-188), with every
- * touched expert's weights read once per task of its (token, pick) pairs on
- * int8 MFMA: IQ2_XXS gate/up + IQ2_XS down layers always, layers of other or
- * mixed types from 13 tokens on (below, one layer call per token). Needs a context opened with max_tokens >= T; picks
+ * then warm_execute's fixed-order combine, runtime.cpp:180-188) but for the
+ * order of the float sums over a row's blocks, with every touched expert's
+ * weights read once per task of its (token, pick) pairs on int8 MFMA: IQ2_XXS
+ * gate/up + IQ2_XS down layers always, layers of other or mixed types from 13
+ * tokens on (below, one layer call per token, with that call's bits). The bits
+ * of a token do not depend on the other tokens of a call served by the same
+ * kernels. Needs a context opened with max_tokens >= T; picks
  * of one token unique. The async form takes device pointers and checks ids on
  * the device (a bad id sets the flag; that pick contributes nothing). */
 int32_t xl_grouped_forward(xl_context* ctx, int32_t layer, int32_t T, int32_t k, const int32_t* ids, const float* w,

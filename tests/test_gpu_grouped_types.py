@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 import crosslane_amd as xl
+from perf import cases
 from tests.conftest import max_rel
 
 pytestmark = pytest.mark.gpu
@@ -90,3 +91,26 @@ def test_tasks_of_several_tiles(dim, ff):
         lane.sync()
     assert float(out.abs().max()) > 0
     assert torch.equal(out.view(torch.int32), traced.view(torch.int32))
+
+
+@pytest.mark.parametrize("dim,ff", [(4096, 3072), (5120, 2304), (1024, 512)])
+@pytest.mark.parametrize("kind", ["iq1", "mixed"])
+@pytest.mark.parametrize("T", [64, 160])     # tasks of up to 16 pairs, and of up to 64
+def test_no_further_from_64_bits_than_layer_calls(monkeypatch, kind, dim, ff, T):
+    """A grouped call over IQ1_M or mixed layers replaces the layer calls of its
+    tokens: its tokens' errors against the same arithmetic in 64 bits (the median, which
+    no moved quant of h reaches) are no larger than theirs."""
+    print(f"[gpu-step] error against 64 bits {kind} {dim}x{ff} T={T}", flush=True)
+    case = {"job": "grouped", "dim": dim, "ff": ff, "experts": 48, "kind": kind, "tokens": T, "picks": 6, "limit": 0.0,
+            "routed": False}
+    want = cases.exact(case, 1)["out"].cuda()
+    err = {}
+    for path in ("0", "1"):                  # layer calls, grouped kernels
+        monkeypatch.setenv("XL_GROUPED_PATH", path)
+        s = cases.prepare(case, 1)
+        with s["lane"]:
+            out = cases.run(s)["out"]
+            torch.cuda.synchronize()
+            err[path] = float(((out.double() - want).norm(dim=1) / want.norm(dim=1)).median())
+    print(f"layer calls {err['0']:.3e}, grouped {err['1']:.3e}", flush=True)
+    assert err["1"] <= err["0"]
