@@ -31,8 +31,8 @@
 // more MFMAs on those sums (11 bits, split 16 hi + lo by the quantizer).
 //
 // Work: a wave takes one tile at a time, two streams of 16 rows that share the
-// activations (gate and up rows, or 32 down rows), from its workgroup's current
-// bundle; a wave that finds the bundle empty fetches the next one from the
+// activations (gate and up rows, or 32 down rows; 16 where tiles are few), from its
+// workgroup's current bundle; a wave that finds the bundle empty fetches the next one from the
 // device's queue of the type. Waves never wait for each other inside a type (a
 // workgroup barrier per item left every wave waiting for the item's chain of
 // dependent loads: task, matrix, scales, weights). A layer of several types has
@@ -60,6 +60,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "xl_dev.hpp"
@@ -74,12 +75,19 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 constexpr int kTile = 16;   // pairs per tile (the MFMA M dimension)
 // GroupArgs::pos: slot of a pair, and whether its x / h go there in the IQ1_M order.
 constexpr int kSlotX1 = 1 << 30, kSlotH1 = 1 << 29, kSlotMask = kSlotH1 - 1;
-// Pairs per expert from which tasks hold up to 64 pairs, in kernels of 8 waves (2 per
-// SIMD: their registers). 4096 x 3072, 384 experts, IQ2: 12 per expert 1,582 us, 32
-// per expert 2,341 us (3,075 by 16-pair tasks); 11 per expert 1,587 against 1,548, 8
-// per expert 1,528 against 1,449. Also where a workgroup has at most 8 tiles: 12 waves
-// would share them (1024 x 512, 64 experts, 64 tokens: 46.0 against 51.8 us).
-constexpr int kMultiPairs = 12;
+// Tasks hold up to 64 pairs, in kernels of 8 waves (2 per SIMD: their registers), from
+// kMultiPairs pairs per expert on (several types: kMultiPairsMix) if that leaves more
+// than kMultiTiles tiles per workgroup, or half of them and four times the pairs. 4096
+// x 3072, 384 experts, IQ2: 12 per expert 1,582 us, 32 per expert 2,341 us (3,075 by
+// 16-pair tasks); 11 per expert 1,587 against 1,548, 8 per expert 1,528 against 1,449.
+// With few tiles the pairs of a task are a chain that idle waves could have shared: 256
+// tokens of one pick over 8 experts (6 tiles) 104.6 us against 94.5, 1024 x 512, 64
+// tokens of 8 over 8 experts (1 tile) 45.0 against 40.1, but 512 tokens there (8 tiles)
+// 69.7 against 103.1, and 5120 x 2304, 512 tokens of one over 8 (5 tiles, 64 per expert)
+// 129.2 against 158.1. Several types: 12 per expert 357 against 347 us, 24 454 and 502.
+// IQ1_M decodes faster and gains earlier: 128 tokens of 2 over 8 experts (6 tiles) 84.1
+// against 96.9, 5120 x 2304, 32 of 6 over 8 (5 tiles) 76.0 against 81.0.
+constexpr int kMultiPairs = 12, kMultiPairsMix = 16, kMultiTiles = 6, kMultiTilesIQ1 = 4;
 // Relative cost of a tile by type (XXS, XS, IQ1_M), for the first share of a mixed
 // layer's workgroups (the queues even out what it misses).
 __device__ constexpr int kTileCost[3] = {10, 11, 8};
@@ -598,24 +606,26 @@ __device__ __forceinline__ void products1(const Dec& w, const Act<kIQ1_M>& x, in
 #pragma unroll
     for (int r = 0; r < RR; ++r) bi[r] = 8 * M[r] + (16 * Hs[r] + L[r]);
 }
-// Block integers of the two IQ2 streams, bi[s][r], r < RR: exact.
-template <int TY, int RR>
-__device__ __forceinline__ void products(const Dec (&w)[2], const Act<TY>& x, uint32_t mk, int (&bi)[2][4]) {
+// Block integers of the NS IQ2 streams, bi[s][r], r < RR: exact.
+template <int TY, int RR, int NS>
+__device__ __forceinline__ void products(const Dec (&w)[NS], const Act<TY>& x, uint32_t mk, int (&bi)[NS][4]) {
     // each step's MFMA is issued before the previous step's multiply-adds read theirs
-    v4i C[16], C1[TY == kIQ2_XS ? 16 : 1];
+    v4i C[8 * NS], C1[TY == kIQ2_XS ? 8 * NS : 1];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) bi[0][r] = bi[1][r] = 0;
+    for (int s = 0; s < NS; ++s)
 #pragma unroll
-    for (int i = 0; i <= 16; ++i) {
-        if (i < 16) {
-            const long A = act8<TY>(x, i >> 1);
-            C[i] = mfma(A, w[i & 1].B[i >> 1], v4i{0, 0, 0, 0});
+        for (int r = 0; r < 4; ++r) bi[s][r] = 0;
+#pragma unroll
+    for (int i = 0; i <= 8 * NS; ++i) {
+        if (i < 8 * NS) {
+            const long A = act8<TY>(x, i / NS);
+            C[i] = mfma(A, w[i % NS].B[i / NS], v4i{0, 0, 0, 0});
             // entries 2, 3 masked out (lanes e4 >= 2 hold them on both sides)
             if constexpr (TY == kIQ2_XS)
-                C1[i] = mfma(pack64(uint32_t(uint64_t(A)) & mk, uint32_t(uint64_t(A) >> 32) & mk), w[i & 1].B[i >> 1], v4i{0, 0, 0, 0});
+                C1[i] = mfma(pack64(uint32_t(uint64_t(A)) & mk, uint32_t(uint64_t(A) >> 32) & mk), w[i % NS].B[i / NS], v4i{0, 0, 0, 0});
         }
         if (i > 0) {
-            const int s = (i - 1) & 1, c = (i - 1) >> 1;
+            const int s = (i - 1) % NS, c = (i - 1) / NS;
             if constexpr (TY == kIQ2_XS) {   // ls1 C1 + ls2 (C - C1) as ls2 C + (ls1 - ls2) C1, exactly
                 const int ls2 = int(__builtin_amdgcn_ubfe(w[s].s[c >> 2], 8 * (c & 3), 8));
                 const int dls = __builtin_amdgcn_sbfe(int(w[s].s[2 + (c >> 2)]), 8 * (c & 3), 8);
@@ -631,7 +641,7 @@ __device__ __forceinline__ void products(const Dec (&w)[2], const Act<TY>& x, ui
 }
 
 // ---------------------------------------------------------------------------
-// Tiles. GU: rows 16 tl .. + 15 of gate and of up; down: rows 32 tl .. + 31.
+// Tiles. GU: rows 16 tl .. + 15 of gate and of up; down: 16 NS rows from 16 NS tl on.
 // ---------------------------------------------------------------------------
 // LDS written by one wave and read by its other lanes.
 __device__ __forceinline__ void wave_sync() {
@@ -659,27 +669,22 @@ __device__ __forceinline__ void next_chain(float* acc, float* total, int b, int 
     }
 }
 // TR: also write each pair's block integers (GroupArgs::tint).
-template <bool GU, int TY, bool TR, bool DB, bool F8>
+template <bool GU, int TY, bool TR, bool DB, bool F8, int NS>
 __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int tl, uint8_t* lds, uint8_t* wl, int lane,
                                         uint32_t& sunk) {
     const int col = lane & 15, e4 = lane >> 4, nb = (GU ? a.dim : a.ff) / 256;
     const uint32_t mk = e4 < 2 ? ~0u : 0u;   // lanes of entries 0, 1
-    Stream st[2];
-    const uint8_t* planes[2];   // fp16 scales of the streams' rows
-    if constexpr (GU) {
+    static_assert(!GU || NS == 2, "gate and up");
+    Stream st[NS];
+    const uint8_t* planes[NS];   // fp16 scales of the streams' rows
+    uint32_t row0nb[NS];
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const MatRef m = mat_at(a.descs, tk.x, s);
-            st[s] = Stream{rsrc(m.base), uint32_t(16 * tl + col) * uint32_t(nb), uint32_t(m.off1), uint32_t(m.off2)};
-            planes[s] = m.base + (TY == kIQ2_XXS ? m.off1 : m.off2) + size_t(16 * tl) * nb * 2;
-        }
-    } else {
-        const MatRef m = mat_at(a.descs, tk.x, 2);
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            st[s] = Stream{rsrc(m.base), uint32_t(32 * tl + 16 * s + col) * uint32_t(nb), uint32_t(m.off1), uint32_t(m.off2)};
-            planes[s] = m.base + (TY == kIQ2_XXS ? m.off1 : m.off2) + size_t(32 * tl + 16 * s) * nb * 2;
-        }
+    for (int s = 0; s < NS; ++s) {
+        const MatRef m = mat_at(a.descs, tk.x, GU ? s : 2);
+        const int row0 = GU ? 16 * tl : 16 * (NS * tl + s);
+        row0nb[s] = uint32_t(row0 * nb);
+        st[s] = Stream{rsrc(m.base), uint32_t((row0 + col) * nb), uint32_t(m.off1), uint32_t(m.off2)};
+        planes[s] = m.base + (TY == kIQ2_XXS ? m.off1 : m.off2) + size_t(row0) * nb * 2;
     }
     // A operand: slot col of the tile (past its pairs: unused slot memory, whose
     // outputs are discarded), the lane's chunk e4
@@ -691,19 +696,18 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
         for (int i = 0; i < 4; ++i) x.a[i] = ld128(rx, va + 4096u * blk + 1024u * i);
         if constexpr (TY == kIQ1_M) x.a[4] = ld128(rx, va + 1024u * blk, 4096u * nb);
     };
-    Raw w0[2], w1[2];   // IQ2
+    Raw w0[NS], w1[NS];   // IQ2
     uint32_t t0 = 0, t2 = 0;
-    auto load = [&](Raw (&w)[2], Act<TY>& x, int blk) {
+    auto load = [&](Raw (&w)[NS], Act<TY>& x, int blk) {
 #pragma unroll
-        for (int s = 0; s < 2; ++s) load_raw<TY>(w[s], st[s], blk, e4);
+        for (int s = 0; s < NS; ++s) load_raw<TY>(w[s], st[s], blk, e4);
         load_x(x, blk);
     };
-    auto touch2 = [&](int blk) { return touch(st[0], blk) ^ touch(st[1], blk); };
-    Raw1 r1[2];         // IQ1_M
-    const uint32_t row0nb[2] = {uint32_t(GU ? 16 * tl : 32 * tl) * uint32_t(nb), uint32_t(GU ? 16 * tl : 32 * tl + 16) * uint32_t(nb)};
+    auto touch2 = [&](int blk) { return touch(st[0], blk) ^ touch(st[NS - 1], blk); };
+    Raw1 r1[NS];         // IQ1_M
     if constexpr (TY == kIQ1_M) {
 #pragma unroll
-        for (int s = 0; s < 2; ++s) load_raw1(r1[s], st[s], row0nb[s], 0, nb, lane);
+        for (int s = 0; s < NS; ++s) load_raw1(r1[s], st[s], row0nb[s], 0, nb, lane);
         if (DB) load_x(x0, 0);
     } else {
         load(w0, x0, 0);
@@ -718,7 +722,7 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
     for (int i = lane; i < 4 * nb; i += 64) reinterpret_cast<float4*>(pd)[i] = pds[i];
     if constexpr (TY != kIQ1_M) {
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
+        for (int s = 0; s < NS; ++s)
             for (int i = lane; i < 2 * nb; i += 64)   // 16 rows x nb halves, 16 B a piece
                 reinterpret_cast<uint4*>(rd + 16 * kGrpNb * s)[i] = reinterpret_cast<const uint4*>(planes[s])[i];
     }
@@ -731,28 +735,28 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
     wave_sync();
     // RR: output registers that can hold a pair (ceil(pairs / 4), rounded up to 2 or 4)
     auto run = [&]<int RR>() {
-        float acc[2][4] = {}, total[2][4];
+        float acc[NS][4] = {}, total[NS][4];
         int blk_c = 0;   // block the next compute() handles
-        auto compute = [&](const Raw (&w)[2], const Act<TY>& x) {
+        auto compute = [&](const Raw (&w)[NS], const Act<TY>& x) {
             const int b = blk_c++;
-            Dec dec[2];
-            int bi[2][4];
+            Dec dec[NS];
+            int bi[NS][4];
             if constexpr (TY == kIQ1_M) {
 #pragma unroll
-                for (int s = 0; s < 2; ++s) {   // one stream after the other: both at once spill
+                for (int s = 0; s < NS; ++s) {   // one stream after the other: both at once spill
                     decode<TY>(dec[s], w[s], lds, lane, e4);
                     products1<RR>(dec[s], x, bi[s]);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             } else {
 #pragma unroll
-                for (int s = 0; s < 2; ++s) decode<TY>(dec[s], w[s], lds, lane, e4);
-                products<TY, RR>(dec, x, mk, bi);
+                for (int s = 0; s < NS; ++s) decode<TY>(dec[s], w[s], lds, lane, e4);
+                products<TY, RR, NS>(dec, x, mk, bi);
             }
             if constexpr (TR) {   // pair po[r]'s block integers of this lane's rows
                 const size_t gu = size_t(a.ff) * (a.dim / 256), rec = 2 * gu + size_t(a.dim) * (a.ff / 256);
 #pragma unroll
-                for (int s = 0; s < 2; ++s)
+                for (int s = 0; s < NS; ++s)
 #pragma unroll
                     for (int r = 0; r < RR; ++r)
                         if (a.tint && po[r] >= 0)
@@ -761,7 +765,7 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
             const float4 xd4 = *reinterpret_cast<const float4*>(pd + 16 * b + 4 * e4);
             const float xd[4] = {xd4.x, xd4.y, xd4.z, xd4.w};
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
+            for (int s = 0; s < NS; ++s) {
                 const float d = TY == kIQ1_M ? dec[s].d : h2f(rd[16 * kGrpNb * s + col * nb + b]);
 #pragma unroll
                 for (int r = 0; r < RR; ++r) acc[s][r] = fmaf(__fmul_rn(d, xd[r]), float(bi[s][r]), acc[s][r]);
@@ -772,13 +776,13 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
             // meanwhile
             uint8_t* raw = wl + 64 * kGrpNb;
             for (int b = 0; b < nb; b += 4) {
-                if (b > 0) next_chain<F8, 8>(acc[0], total[0], b, nb);
+                if (b > 0) next_chain<F8, 4 * NS>(acc[0], total[0], b, nb);
                 wave_sync();   // the previous four are read
 #pragma unroll
-                for (int s = 0; s < 2; ++s) store_raw1(raw + kRaw1 * s, r1[s], lane);
+                for (int s = 0; s < NS; ++s) store_raw1(raw + kRaw1 * s, r1[s], lane);
                 wave_sync();
 #pragma unroll
-                for (int s = 0; s < 2; ++s) load_raw1(r1[s], st[s], row0nb[s], min(b + 4, nb - 1), nb, lane);
+                for (int s = 0; s < NS; ++s) load_raw1(r1[s], st[s], row0nb[s], min(b + 4, nb - 1), nb, lane);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     Act<TY>& now = DB && (i & 1) ? x1 : x0;
@@ -787,9 +791,9 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
                     if (b + i < nb) {
                         if (!DB) load_x(now, b + i);   // under the first stream's decode (a second set spills)
                         __builtin_amdgcn_sched_barrier(0);
-                        Raw w[2];
+                        Raw w[NS];
 #pragma unroll
-                        for (int s = 0; s < 2; ++s) read_raw1(w[s], raw + kRaw1 * s, i, col, e4);
+                        for (int s = 0; s < NS; ++s) read_raw1(w[s], raw + kRaw1 * s, i, col, e4);
                         compute(w, now);
                     }
                 }
@@ -799,7 +803,7 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
             // so no wait ever covers a load issued in the same step); line touches four
             // blocks ahead in fixed registers, one per line of two blocks.
             for (int b = 0; b < nb; b += 4) {
-                if (b > 0) next_chain<F8, 8>(acc[0], total[0], b, nb);
+                if (b > 0) next_chain<F8, 4 * NS>(acc[0], total[0], b, nb);
                 load(w1, x1, min(b + 1, nb - 1));
                 sink(sunk, t0);
                 t0 = touch2(min(b + 5, nb - 1));
@@ -819,7 +823,7 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
             }
             sink(sunk, t0 ^ t2);
         }
-        next_chain<F8, 8>(acc[0], total[0], 0, nb);
+        next_chain<F8, 4 * NS>(acc[0], total[0], 0, nb);
 #pragma unroll
         for (int r = 0; r < RR; ++r)
             if (po[r] >= 0) {
@@ -827,9 +831,9 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
                     a.h[size_t(po[r]) * a.ff + 16 * tl + col] =
                         silu_mul3(__fmul_rn(0.125f, acc[0][r]), __fmul_rn(0.125f, acc[1][r]), a.lim);
                 } else {
-                    float* y = a.y + size_t(po[r]) * a.dim + 32 * tl + col;
-                    y[0] = __fmul_rn(0.125f, acc[0][r]);
-                    y[16] = __fmul_rn(0.125f, acc[1][r]);
+                    float* y = a.y + size_t(po[r]) * a.dim + 16 * NS * tl + col;
+#pragma unroll
+                    for (int s = 0; s < NS; ++s) y[16 * s] = __fmul_rn(0.125f, acc[s][r]);
                 }
             }
     };
@@ -918,7 +922,7 @@ __device__ __forceinline__ void do_tiles(const GroupArgs& a, const int4& tk, int
 #pragma unroll
                 for (int s = 0; s < 2; ++s) products1<4>(dec[s], now.x, bi[s]);
             } else {
-                products<TY, 4>(dec, now.x, mk, bi);
+                products<TY, 4, 2>(dec, now.x, mk, bi);
             }
             const float xd[4] = {__uint_as_float(now.d.x), __uint_as_float(now.d.y), __uint_as_float(now.d.z), __uint_as_float(now.d.w)};
 #pragma unroll
@@ -984,15 +988,15 @@ __device__ __forceinline__ void do_tiles(const GroupArgs& a, const int4& tk, int
 }
 
 // MASK: block types among the launch's matrices (bits 1 IQ2_XXS, 2 IQ2_XS, 4 IQ1_M).
-// MT: tasks may hold up to 16 MT pairs.
+// MT: tasks may hold up to 16 MT pairs. NS: streams per tile (down of 16 or 32 rows).
 // F8: the order of the float sums (do_tile).
-template <bool GU, int MASK, int NW, int MT, bool TR, bool F8>
+template <bool GU, int MASK, int NW, int MT, bool TR, bool F8, int NS = 2>
 __global__ __launch_bounds__(NW * 64, 1) void grouped_kernel(GroupArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[grp_lds_bytes(MASK, NW)];
     __shared__ uint32_t s_bundle;   // current bundle << 8 | its next tile
     __shared__ int s_open;
     const int t = threadIdx.x, lane = t & 63, wv = uni(t >> 6);
-    const int tiles = GU ? a.ff / 16 : a.dim / 32;   // per task
+    const int tiles = GU ? a.ff / 16 : a.dim / (16 * NS);   // per task
     int n[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) n[i] = uni(GU ? a.queue->gu_tasks[i] : a.queue->dn_tasks[i]);
@@ -1035,9 +1039,9 @@ __global__ __launch_bounds__(NW * 64, 1) void grouped_kernel(GroupArgs a) {
                 const int task = ft / tiles, tl = ft - task * tiles, nb = (GU ? a.dim : a.ff) / 256;
                 const int4 tk = task_at((GU ? a.tasks : a.dtasks) + base, task);
 #pragma unroll
-                for (int s = 0; s < 2; ++s) {
+                for (int s = 0; s < NS; ++s) {
                     const MatRef m = mat_at(a.descs, tk.x, GU ? s : 2);
-                    const int row = (GU ? 16 * tl : 32 * tl + 16 * s) + (lane & 15);
+                    const int row = (GU ? 16 * tl : 16 * (NS * tl + s)) + (lane & 15);
                     warm[s] = ld32(rsrc(m.base), (ti == 2 ? 32u : 64u) * uint32_t(row * nb));
                 }
             }
@@ -1074,7 +1078,7 @@ __global__ __launch_bounds__(NW * 64, 1) void grouped_kernel(GroupArgs a) {
             const int4 tk = task_at((GU ? a.tasks : a.dtasks) + base, task);
             const auto tile_of = [&]<int TY>() {
                 if constexpr (MT == 1) {
-                    do_tile<GU, TY, TR, NW <= 8, F8>(a, tk, tl, lds, wl, lane, sunk);
+                    do_tile<GU, TY, TR, NW <= 8, F8, NS>(a, tk, tl, lds, wl, lane, sunk);
                 } else {
                     if (tk.z <= 16) do_tiles<GU, TY, 1, F8>(a, tk, tl, lds, wl, lane, sunk);
                     else if (tk.z <= 32) do_tiles<GU, TY, 2, F8>(a, tk, tl, lds, wl, lane, sunk);
@@ -1144,6 +1148,46 @@ __global__ __launch_bounds__(256) void gcombine_kernel(GroupArgs a) {
     *reinterpret_cast<VT*>(a.out + size_t(tok) * a.dim + c) = acc;
 }
 
+// How a call's tasks and kernels are cut, from what the host knows: T draws of k of
+// the E experts touch E (1 - (1 - k / E)^T) of them. No result depends on it.
+struct GroupPlan {
+    bool multi;      // tasks of up to 64 pairs
+    bool gu8, dn8;   // gate/up, down: the kernels of 8 waves instead of 12
+    bool dn_half;    // down tiles of 16 rows instead of 32, 12 waves
+};
+GroupPlan group_plan(const GroupArgs& a, int gu_types, int dn_types, bool trace, int cus) {
+    GroupPlan p{};
+    if (trace) return p;   // one kernel each
+    const double E = a.n_experts, pairs = double(a.T) * a.k;
+    const double touched = E * (1.0 - std::pow(1.0 - std::min(1.0, a.k / E), a.T));
+    const double gu_tiles = a.ff / 16, dn_tiles = a.dim / 32;   // per task
+    const auto per_wg = [&](double tasks, double tiles) { return tasks * tiles / cus; };
+    const auto mixed = [](int types) { return types != 1 && types != 2 && types != 4; };
+    const int least = mixed(gu_types) || mixed(dn_types) ? kMultiPairsMix : kMultiPairs;
+    const double wide = per_wg(std::max(touched, pairs / 64), std::max(gu_tiles, dn_tiles));
+    const bool iq2 = gu_types == 1 && dn_types == 2;
+    p.multi = pairs >= least * E && (wide > (iq2 || least == kMultiPairsMix ? kMultiTiles : kMultiTilesIQ1) ||
+                                     (wide >= kMultiTiles / 2 && pairs >= 4 * least * E));
+    p.gu8 = p.dn8 = p.multi;
+    if (p.multi) return p;
+    if (!iq2) {   // where 12 waves would share at most 8 tiles
+        p.gu8 = p.dn8 = per_wg(std::min(pairs, E), std::max(gu_tiles, dn_tiles)) <= 8;
+        return p;
+    }
+    // IQ2_XXS / IQ2_XS, tiles per workgroup, each way timed over five shapes, 8 to 384
+    // experts and 1 to 512 tokens. Gate/up: 8 waves to 8 tiles (0.90 to 1.00 of 12 waves'
+    // call); from there 12 to 24, past which the tiles come from a queue, one bundle at a
+    // time: 1.01 to 1.05 the other way; past 24 rows of four blocks are faster on 8 waves
+    // (0.97), and long rows to 36 tiles (0.95 to 0.99), the rest on 12 (1.00 to 1.04).
+    // Down: tiles of 16 rows to 12 tiles (0.87 to 1.00; past them 1.02 to 1.2), with rows of
+    // two blocks to 6, where 8 waves follow to 16 and past 24 (0.92 to 1.0).
+    const double tasks = std::max(touched, pairs / 16), gu = per_wg(tasks, gu_tiles), dn = per_wg(tasks, dn_tiles);
+    p.gu8 = gu <= 8 || (gu > 24 && (a.dim <= 1024 || (a.dim > 2048 && gu <= 36)));
+    p.dn_half = dn <= (a.ff <= 512 ? 6 : 12);
+    p.dn8 = !p.dn_half && a.ff <= 512 && (dn <= 16 || dn > 24);
+    return p;
+}
+
 }  // namespace
 
 hipError_t launch_grouped(GroupArgs args, int gu_types, int dn_types, int cus, hipStream_t s) {
@@ -1155,15 +1199,18 @@ hipError_t launch_grouped(GroupArgs args, int gu_types, int dn_types, int cus, h
         return hipErrorNotSupported;
     const bool trace = args.tq8x || args.tq8h || args.th || args.tint, iq2 = gu_types == 1 && dn_types == 2;
     if (trace && !iq2) return hipErrorNotSupported;
-    const int64_t pairs = int64_t(args.T) * args.k, experts = pairs < args.n_experts ? pairs : args.n_experts;
-    const bool multi = !trace && (pairs >= int64_t(kMultiPairs) * args.n_experts ||
-                                  experts * std::max(args.ff / 16, args.dim / 32) <= 8 * int64_t(cus));
-    args.cap = multi ? 64 : 16;
+    const GroupPlan plan = group_plan(args, gu_types, dn_types, trace, cus);
+    args.cap = plan.multi ? 64 : 16;
     const int P = args.T * args.k, nbx = args.dim / 256, nbh = args.ff / 256;
     const auto grouped = [&](auto kernel, int nw = 12) { hipLaunchKernelGGL(kernel, dim3(cus), dim3(nw * 64), 0, s, args); };
     const auto rows = [&](auto kernel, const float* src, int n, int nb, int8_t* q, float* d, uint8_t* tr) {
         hipLaunchKernelGGL(kernel, dim3((n * nb + 3) / 4), dim3(256), 0, s, src, n, nb, q, d, args.pos, args.k, args.err, tr);
     };
+    // sums by eights (next_chain), where a row has more than eight blocks: without, it is
+    // one chain all the same, and several-type kernels spill less (1024 x 512, 256 tokens
+    // of 6 over 64 experts 97.9 to 93.1 us)
+    const bool gu_f8 = !iq2 && nbx > 8, dn_f8 = !iq2 && nbh > 8;
+    const auto sums = [&](bool f8, auto chain, auto eights, int nw) { grouped(f8 ? eights : chain, nw); };
     // the queues start past the workgroups' own first bundles (launches of one type)
     args.gu_first = gu_types == 1 || gu_types == 4 ? cus : 0;
     args.dn_first = dn_types == 2 || dn_types == 4 ? cus : 0;
@@ -1176,35 +1223,29 @@ hipError_t launch_grouped(GroupArgs args, int gu_types, int dn_types, int cus, h
     } else {
         rows(gu_types & 4 ? q8k_rows_kernel<ROWS_X, true, false> : q8k_rows_kernel<ROWS_X, false, false>, args.x, args.T, nbx,
              args.xq, args.xd, nullptr);
-        if (multi) {
-            if (iq2) grouped(grouped_kernel<true, 1, 8, 4, false, false>, 8);
-            else if (gu_types == 1) grouped(grouped_kernel<true, 1, 8, 4, false, true>, 8);
-            else if (gu_types == 4) grouped(grouped_kernel<true, 4, 8, 4, false, true>, 8);
-            else grouped(grouped_kernel<true, 7, 8, 4, false, true>, 8);
-        } else if (iq2) {
-            grouped(grouped_kernel<true, 1, NW, 1, false, false>);
-        } else if (gu_types == 1) {
-            grouped(grouped_kernel<true, 1, NW, 1, false, true>);
+        if (gu_types == 1) {
+            if (plan.gu8) sums(gu_f8, grouped_kernel<true, 1, 8, 4, false, false>, grouped_kernel<true, 1, 8, 4, false, true>, 8);
+            else sums(gu_f8, grouped_kernel<true, 1, NW, 1, false, false>, grouped_kernel<true, 1, NW, 1, false, true>, NW);
         } else if (gu_types == 4) {
-            grouped(grouped_kernel<true, 4, NW, 1, false, true>);
+            if (plan.gu8) sums(gu_f8, grouped_kernel<true, 4, 8, 4, false, false>, grouped_kernel<true, 4, 8, 4, false, true>, 8);
+            else sums(gu_f8, grouped_kernel<true, 4, NW, 1, false, false>, grouped_kernel<true, 4, NW, 1, false, true>, NW);
         } else {
-            grouped(grouped_kernel<true, 7, NWM, 1, false, true>, NWM);
+            if (plan.multi) sums(gu_f8, grouped_kernel<true, 7, NWM, 4, false, false>, grouped_kernel<true, 7, NWM, 4, false, true>, NWM);
+            else sums(gu_f8, grouped_kernel<true, 7, NWM, 1, false, false>, grouped_kernel<true, 7, NWM, 1, false, true>, NWM);
         }
         rows(dn_types & 4 ? q8k_rows_kernel<ROWS_H, true, false> : q8k_rows_kernel<ROWS_H, false, false>, args.h, P, nbh,
              args.hq, args.hd, nullptr);
-        if (multi) {
-            if (iq2) grouped(grouped_kernel<false, 2, 8, 4, false, false>, 8);
-            else if (dn_types == 2) grouped(grouped_kernel<false, 2, 8, 4, false, true>, 8);
-            else if (dn_types == 4) grouped(grouped_kernel<false, 4, 8, 4, false, true>, 8);
-            else grouped(grouped_kernel<false, 7, 8, 4, false, true>, 8);
-        } else if (iq2) {
-            grouped(grouped_kernel<false, 2, NW, 1, false, false>);
+        if (plan.dn_half) {   // IQ2 layers only
+            grouped(grouped_kernel<false, 2, NW, 1, false, false, 1>);
         } else if (dn_types == 2) {
-            grouped(grouped_kernel<false, 2, NW, 1, false, true>);
+            if (plan.dn8) sums(dn_f8, grouped_kernel<false, 2, 8, 4, false, false>, grouped_kernel<false, 2, 8, 4, false, true>, 8);
+            else sums(dn_f8, grouped_kernel<false, 2, NW, 1, false, false>, grouped_kernel<false, 2, NW, 1, false, true>, NW);
         } else if (dn_types == 4) {
-            grouped(grouped_kernel<false, 4, NW, 1, false, true>);
+            if (plan.dn8) sums(dn_f8, grouped_kernel<false, 4, 8, 4, false, false>, grouped_kernel<false, 4, 8, 4, false, true>, 8);
+            else sums(dn_f8, grouped_kernel<false, 4, NW, 1, false, false>, grouped_kernel<false, 4, NW, 1, false, true>, NW);
         } else {
-            grouped(grouped_kernel<false, 7, NWM, 1, false, true>, NWM);
+            if (plan.multi) sums(dn_f8, grouped_kernel<false, 7, NWM, 4, false, false>, grouped_kernel<false, 7, NWM, 4, false, true>, NWM);
+            else sums(dn_f8, grouped_kernel<false, 7, NWM, 1, false, false>, grouped_kernel<false, 7, NWM, 1, false, true>, NWM);
         }
     }
     const bool al16 = (reinterpret_cast<uintptr_t>(args.out) | reinterpret_cast<uintptr_t>(args.shared)) % 16 == 0;

@@ -114,3 +114,37 @@ def test_no_further_from_64_bits_than_layer_calls(monkeypatch, kind, dim, ff, T)
             err[path] = float(((out.double() - want).norm(dim=1) / want.norm(dim=1)).median())
     print(f"layer calls {err['0']:.3e}, grouped {err['1']:.3e}", flush=True)
     assert err["1"] <= err["0"]
+
+
+@pytest.mark.parametrize("dim,ff,E,T,k", [
+    (1024, 512, 8, 64, 8), (2048, 1024, 64, 4, 6), (2048, 1024, 64, 64, 6), (1024, 512, 64, 64, 7), (1024, 512, 224, 64, 7),
+    (4096, 3072, 8, 20, 6), (256, 256, 8, 256, 8), (768, 4096, 6, 50, 4), (2304, 2048, 40, 1, 8), (1024, 512, 8, 512, 8)])
+def test_plans_keep_the_bits(dim, ff, E, T, k):
+    """However a call's tiles are cut (waves per workgroup, down rows per tile, pairs
+    per task: by the work that the host expects), an IQ2 call has the bits of the
+    traced one, which is always cut the same way."""
+    print(f"[gpu-step] plans {dim}x{ff} E={E} T={T} k={k}", flush=True)
+    rng = np.random.default_rng(dim + E + T)
+    types = np.zeros((1, E, 3), np.int32)
+    types[..., :2], types[..., 2] = 16, 17
+    ids = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)
+    if T > 1:
+        ids[T // 2] = -1                        # a token without a valid pick: the shared row alone
+    args = [torch.from_numpy(a).cuda() for a in (ids, rng.random((T, k)).astype(np.float32),
+                                                 rng.standard_normal((T, dim)).astype(np.float32))]
+    out, traced = torch.zeros((T, dim), device="cuda"), torch.zeros((T, dim), device="cuda")
+    q8x = torch.zeros(T * (dim // 256) * 292, dtype=torch.uint8, device="cuda")
+    shared = torch.from_numpy(rng.standard_normal((T, dim)).astype(np.float32)).cuda()
+    torch.cuda.synchronize()
+    with xl.Lane(dim, ff, 1, E, types, max_picks=8, max_tokens=T) as lane:
+        lane.generate(seed=9)
+        lane.grouped_forward_async(0, *args, out, shared=shared)
+        lane.grouped_trace_async(0, *args, traced, q8x=q8x, shared=shared)
+        if T > 1:
+            with pytest.raises(xl.XLError, match="expert id"):
+                lane.sync()
+        else:
+            lane.sync()
+    assert int((out.view(torch.int32) != traced.view(torch.int32)).sum()) == 0
+    assert T == 1 or int((out[T // 2] != shared[T // 2]).sum()) == 0
+    assert float(out.abs().max()) > 0
