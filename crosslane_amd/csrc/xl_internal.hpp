@@ -283,7 +283,8 @@ hipError_t launch_swiglu_quant32(const float* g, const float* u, int rows, int k
 // Shared-expert FFN of T tokens over dense matrices (xl_shared.hip), with the
 // bits of quant32, mv32, swiglu_quant32 and mv32 run token by token; xq, hq: T x
 // dim and T x ff bytes, xd, hd: a float per 32 of them. hipErrorNotSupported
-// below kFfnTokensMin tokens or for another block type.
+// below kFfnTokensMin tokens, for another block type, or where the row kernels are
+// faster (rows_faster).
 // Two tokens are still faster by the row kernels (29.5 against 34.8 us at 4096 x
 // 3072 of Q5_K / Q6_K; three: 36.6 against 35.3).
 constexpr int kFfnTokensMin = 3;

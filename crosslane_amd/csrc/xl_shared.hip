@@ -497,13 +497,26 @@ __global__ __launch_bounds__(512, 4) void ffn_dn_kernel(const uint8_t* __restric
     }
 }
 
+// Few tokens of a small FFN, where the row kernels' many short rows fill the chip
+// better than a few tiles whose blocks come one after the other. Timed both ways at 2 to
+// 12 tokens over dim 256 .. 5120, ff 256 .. 6144 and four type sets: 3 tokens, ff up to
+// 512 (rows of 2,048 on 1,024; Q8_0, cheaper to decode: 256) 0.99 to 1.10 of the row kernels' time (4096 x 256
+// 26.0 against 24.8 us, 512 x 256 18.9 against 17.1), ff of 2048 0.80 to 0.99; 4 tokens of
+// up to 2^18 weights a matrix 1.01 to 1.11; to 8 of 256 x 256 1.02 to 1.06. Two tokens are
+// faster by rows almost everywhere (kFfnTokensMin), 5120 x 512 from three on by tiles.
+bool rows_faster(int T, int dim, int ff, bool q8) {
+    if (T == 3) return ff <= (q8 ? 256 : dim >= 2048 ? 1024 : 512) && dim < 5120;
+    if (T == 4) return q8 ? ff <= 256 && dim <= 512 : ff <= 512 && dim * ff <= 1 << 18;
+    return T <= 8 && !q8 && dim * ff <= 1 << 16;
+}
+
 }  // namespace
 
 hipError_t launch_ffn_tokens(const MatRef& gate, const MatRef& up, const MatRef& down, int T, int dim, int ff,
                              const float* x, float* out, int8_t* xq, float* xd, int8_t* hq, float* hd, float lim,
                              int* err, int cus, hipStream_t s) {
     if (T < kFfnTokensMin || !dense_type(gate.type) || up.type != gate.type || !dense_type(down.type) || dim % 256 ||
-        ff % 256)
+        ff % 256 || rows_faster(T, dim, ff, gate.type == kQ8_0))
         return hipErrorNotSupported;
     const int nb = dim / 256, t16 = (T + 15) / 16, t32 = (T + 31) / 32, out16 = reinterpret_cast<uintptr_t>(out) % 16 == 0;
     hipLaunchKernelGGL(quant32t_kernel, dim3((T * nb + 3) / 4), dim3(256), 0, s, x, T, dim, xq, xd, err,

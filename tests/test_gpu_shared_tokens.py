@@ -22,7 +22,11 @@ def dev(a):
 @pytest.mark.parametrize("types,dim,ff,T,lim", [
     ((13, 13, 14), 4096, 3072, 16, 0.0), ((13, 13, 14), 4096, 256, 33, 7.0), ((14, 14, 13), 256, 2304, 17, 0.0),
     ((12, 12, 8), 768, 512, 3, 10.0), ((8, 8, 12), 5120, 1280, 47, 7.0), ((14, 14, 12), 4096, 3072, 96, 0.0), ((13, 8, 14), 1024, 768, 32, 0.0),
-    ((12, 14, 8), 2304, 256, 65, 0.0)])
+    ((12, 14, 8), 2304, 256, 65, 0.0),
+    # three to eight tokens on both sides of the line to the row kernels
+    ((12, 12, 8), 768, 2048, 3, 10.0), ((13, 13, 14), 5120, 256, 3, 0.0), ((13, 13, 14), 4096, 512, 3, 0.0),
+    ((8, 8, 8), 1024, 512, 3, 0.0), ((14, 14, 14), 512, 512, 4, 7.0), ((14, 14, 14), 768, 512, 4, 0.0),
+    ((12, 12, 12), 256, 256, 8, 0.0), ((12, 12, 12), 256, 256, 9, 0.0)])
 def test_tokens_equal_single_calls(types, dim, ff, T, lim):
     print(f"[gpu-step] shared FFN types={types} dim={dim} ff={ff} T={T}", flush=True)
     rng = np.random.default_rng(dim + ff + T)
