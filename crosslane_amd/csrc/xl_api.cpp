@@ -181,6 +181,7 @@ struct xl_context {
     struct Group {
         int32_t* ids = nullptr; float* w = nullptr; float* x = nullptr; float* shared = nullptr; float* out = nullptr;
         int8_t* xq = nullptr; float* xd = nullptr;
+        int8_t* xs = nullptr; int8_t* hs = nullptr;   // only for banks with IQ1_M (xl_bank_create)
         int32_t* order = nullptr; int32_t* pos = nullptr; int4* tasks = nullptr; int4* dtasks = nullptr;
         xl::GroupQueue* queue = nullptr;
         float* h = nullptr; int8_t* hq = nullptr; float* hd = nullptr; float* y = nullptr;
@@ -679,7 +680,7 @@ int32_t xl_open(uint32_t abi_version, const xl_config* cfg, xl_context** out, xl
                 {reinterpret_cast<void**>(&g.x), T * dim * 4},
                 {reinterpret_cast<void**>(&g.shared), T * dim * 4},
                 {reinterpret_cast<void**>(&g.out), T * dim * 4},
-                {reinterpret_cast<void**>(&g.xq), slots * dim * 5 / 4},
+                {reinterpret_cast<void**>(&g.xq), slots * dim},
                 {reinterpret_cast<void**>(&g.xd), slots * (dim / 256) * 4},
                 {reinterpret_cast<void**>(&g.order), slots * 4},
                 {reinterpret_cast<void**>(&g.pos), GP * 4},
@@ -687,7 +688,7 @@ int32_t xl_open(uint32_t abi_version, const xl_config* cfg, xl_context** out, xl
                 {reinterpret_cast<void**>(&g.dtasks), tiles * 16},
                 {reinterpret_cast<void**>(&g.queue), sizeof(xl::GroupQueue)},
                 {reinterpret_cast<void**>(&g.h), GP * ff * 4},
-                {reinterpret_cast<void**>(&g.hq), slots * ff * 5 / 4},
+                {reinterpret_cast<void**>(&g.hq), slots * ff},
                 {reinterpret_cast<void**>(&g.hd), slots * (ff / 256) * 4},
                 {reinterpret_cast<void**>(&g.y), GP * dim * 4},
             };
@@ -742,6 +743,8 @@ void xl_close(xl_context* ctx) {
     for (auto* s : ctx->slabs) (void)hipFree(s);
     if (ctx->d_descs) (void)hipFree(ctx->d_descs);
     if (ctx->ws) (void)hipFree(ctx->ws);
+    if (ctx->grp.xs) (void)hipFree(ctx->grp.xs);
+    if (ctx->grp.hs) (void)hipFree(ctx->grp.hs);
     if (ctx->done) (void)hipEventDestroy(ctx->done);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -771,6 +774,19 @@ int32_t xl_bank_create(xl_context* ctx, const int32_t* types, xl_error* err) {
                 ctx->gu_mask[size_t(l)] |= xl::dev::type_bit(types[(size_t(l) * E + e) * 3]);
                 ctx->dn_mask[size_t(l)] |= xl::dev::type_bit(types[(size_t(l) * E + e) * 3 + 2]);
             }
+        // The grouped kernels' sums for IQ1_M matrices, in banks that have them.
+        if (ctx->cfg.max_tokens > 0) {
+            const uint64_t tiles = uint64_t(xl::group_max_tiles(int64_t(ctx->cfg.max_tokens) * ctx->cfg.max_picks, E));
+            const auto sums = [&](const std::vector<int>& masks, int k, int8_t*& p) {
+                if (p || std::none_of(masks.begin(), masks.end(), [](int m) { return (m & 4) != 0; })) return;
+                const uint64_t bytes = xl::align256(4 * tiles * uint64_t(k));
+                const hipError_t e = hipMalloc(&p, bytes);
+                if (e != hipSuccess) fail(XL_E_MEMORY, "grouped IQ1_M sums (%llu bytes): %s", (unsigned long long)bytes, hipGetErrorString(e));
+                ctx->ws_bytes += bytes;
+            };
+            sums(ctx->gu_mask, dim, ctx->grp.xs);
+            sums(ctx->dn_mask, ff, ctx->grp.hs);
+        }
         ctx->descs.assign(size_t(L) * E, xl::ExpertDesc{});
         // One slab per layer, experts contiguous, each matrix's planes 256-B aligned.
         for (int l = 0; l < L; ++l) {
@@ -1130,7 +1146,7 @@ void enqueue_grouped(xl_context* ctx, int32_t layer, int32_t T, int32_t k, const
         a.T = T; a.k = k; a.n_experts = E; a.dim = dim; a.ff = ctx->cfg.ff;
         const auto& g = ctx->grp;
         a.xq = g.xq; a.xd = g.xd; a.order = g.order; a.pos = g.pos; a.tasks = g.tasks; a.dtasks = g.dtasks;
-        a.queue = g.queue;
+        a.queue = g.queue; a.xs = g.xs; a.hs = g.hs;
         a.h = g.h; a.hq = g.hq; a.hd = g.hd; a.y = g.y;
         a.tables = ctx->tables; a.err = ctx->err_flag;
         a.lim = ctx->cfg.swiglu_limit;

@@ -311,13 +311,13 @@ __global__ __launch_bounds__(1024) void bucket_kernel(GroupArgs a) {
 // Q8_K of 256-value blocks of rows, one wave per block, written to the slots of
 // the row's pairs (ROWS_X: a token row goes to its k pairs' slots; ROWS_H: a
 // pair row to its slot; bad ids have none) in the operand order of the MFMA
-// kernels. A tile's slots form one region of nb * 5 KiB; in its first nb * 4 KiB,
-// per block b, the 16-B piece i of chunk e of slot s sits at ((4 b + i) * 4 + e) *
-// 256 + 16 s, so that four lanes of consecutive slots read 64 contiguous bytes.
-// IQ2 order: piece i of chunk e is the 8 quants of entry e of sub-blocks 2i and
-// 2i + 1. IQ1_M order: chunk e is values 64 e .. + 63, piece i 16 of them; then, in
-// the region's last nb KiB, the sums S of each 8 values as S = 16 hi + lo: slot
-// s's 16 bytes at (4 b + e) * 256 + 16 s hold lo, then hi, of chunk e's entries 0, 2,
+// kernels. A tile's slots form one region of nb * 4 KiB, in which, per block b, the
+// 16-B piece i of chunk e of slot s sits at ((4 b + i) * 4 + e) * 256 + 16 s, so that
+// four lanes of consecutive slots read 64 contiguous bytes. IQ2 order: piece i of
+// chunk e is the 8 quants of entry e of sub-blocks 2i and 2i + 1. IQ1_M order: chunk e
+// is values 64 e .. + 63, piece i 16 of them; and in a region of their own, nb KiB per
+// tile (which only banks with IQ1_M have), the sums S of each 8 values as S = 16 hi +
+// lo: slot s's 16 bytes at (4 b + e) * 256 + 16 s hold lo, then hi, of chunk e's entries 0, 2,
 // 4, 6, 1, 3, 5, 7. The block scale goes to the tile's [block][slot] floats.
 // ---------------------------------------------------------------------------
 // The j-th pair of a tile (slot 16 i + j) sits at tile position 4 (j % 4) + j / 4
@@ -325,15 +325,16 @@ __global__ __launch_bounds__(1024) void bucket_kernel(GroupArgs a) {
 // 4 e + r, r = 0..3, gets pairs 4 r + e, so a tile of n pairs has results only
 // in the lanes' first ceil(n / 4) output registers.
 __device__ __forceinline__ int tile_pos(int j) { return ((j & 3) << 2) | (j >> 2); }
-__device__ __forceinline__ size_t tile_off(int tile, int nb) { return size_t(tile) * size_t(nb) * 5120; }
+__device__ __forceinline__ size_t tile_off(int tile, int nb) { return size_t(tile) * size_t(nb) * 4096; }
+__device__ __forceinline__ size_t sum_off(int tile, int nb) { return size_t(tile) * size_t(nb) * 1024; }
 enum { ROWS_X = 0, ROWS_H = 1 };
 // trace (null outside the parity trace): the row's blocks also as 292-byte Q8_K
 // blocks, row-major (a token's for ROWS_X, a pair's for ROWS_H).
 // IQ1: some slots may be in the IQ1_M order.
 template <int MODE, bool IQ1, bool TR>
 __global__ __launch_bounds__(256) void q8k_rows_kernel(const float* __restrict__ src, int rows, int nb,
-                                                       int8_t* __restrict__ q, float* __restrict__ d,
-                                                       const int32_t* __restrict__ pos, int k,
+                                                       int8_t* __restrict__ q, int8_t* __restrict__ sums,
+                                                       float* __restrict__ d, const int32_t* __restrict__ pos, int k,
                                                        int* __restrict__ err, uint8_t* __restrict__ trace) {
     const int b = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (b >= rows * nb) return;   // wave-uniform
@@ -352,7 +353,7 @@ __global__ __launch_bounds__(256) void q8k_rows_kernel(const float* __restrict__
     int sum = __builtin_amdgcn_sdot4(int(r.packed), 0x01010101, 0, false);
     sum += __builtin_amdgcn_update_dpp(0, sum, 0xB1, 0xF, 0xF, false);   // lane ^ 1: the entry's 8 values
     const int j = (lane >> 1) & 7, lo = ((sum + 8) & 15) - 8, hi = (sum - lo) >> 4;
-    const int os = nb * 4096 + (4 * blk + (lane >> 4)) * 256 + (j >> 1) + 4 * (j & 1);
+    const int os = (4 * blk + (lane >> 4)) * 256 + (j >> 1) + 4 * (j & 1);
     const int np = MODE == ROWS_X ? k : 1;
     for (int i = 0; i < np; ++i) {
         const int slot = pos[MODE == ROWS_X ? row * k + i : row];
@@ -362,8 +363,9 @@ __global__ __launch_bounds__(256) void q8k_rows_kernel(const float* __restrict__
         if (IQ1 && (slot & (MODE == ROWS_X ? kSlotX1 : kSlotH1))) {
             *reinterpret_cast<uint32_t*>(t + o1) = r.packed;
             if (!(lane & 1)) {
-                t[os] = int8_t(lo);
-                t[os + 8] = int8_t(hi);
+                int8_t* ts = sums + sum_off(s >> 4, nb) + 16 * tp + os;
+                ts[0] = int8_t(lo);
+                ts[8] = int8_t(hi);
             }
         } else {
             *reinterpret_cast<uint32_t*>(t + o2) = r.packed;
@@ -689,12 +691,13 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
     // A operand: slot col of the tile (past its pairs: unused slot memory, whose
     // outputs are discarded), the lane's chunk e4
     const __amdgpu_buffer_rsrc_t rx = rsrc((GU ? a.xq : a.hq) + tile_off(tk.y >> 4, nb));
+    const __amdgpu_buffer_rsrc_t rs = TY == kIQ1_M ? rsrc((GU ? a.xs : a.hs) + sum_off(tk.y >> 4, nb)) : rx;
     const uint32_t va = 256u * e4 + 16u * col;
     Act<TY> x0, x1;
     auto load_x = [&](Act<TY>& x, int blk) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) x.a[i] = ld128(rx, va + 4096u * blk + 1024u * i);
-        if constexpr (TY == kIQ1_M) x.a[4] = ld128(rx, va + 1024u * blk, 4096u * nb);
+        if constexpr (TY == kIQ1_M) x.a[4] = ld128(rs, va + 1024u * blk);
     };
     Raw w0[NS], w1[NS];   // IQ2
     uint32_t t0 = 0, t2 = 0;
@@ -862,6 +865,7 @@ __device__ __forceinline__ void do_tiles(const GroupArgs& a, const int4& tk, int
         planes[s] = m.base + (TY == kIQ2_XXS ? m.off1 : m.off2) + size_t(row0) * nb * 2;
     }
     const __amdgpu_buffer_rsrc_t rx = rsrc((GU ? a.xq : a.hq) + tile_off(tk.y >> 4, nb));
+    const __amdgpu_buffer_rsrc_t rs = TY == kIQ1_M ? rsrc((GU ? a.xs : a.hs) + sum_off(tk.y >> 4, nb)) : rx;
     const __amdgpu_buffer_rsrc_t rp = rsrc((GU ? a.xd : a.hd) + size_t(tk.y >> 4) * nb * 16);
     const uint32_t va = 256u * e4 + 16u * col;
     struct Step {   // one block's activations and scales of one tile
@@ -870,10 +874,10 @@ __device__ __forceinline__ void do_tiles(const GroupArgs& a, const int4& tk, int
     };
     Step p0, p1;
     auto load_p = [&](Step& p, int blk, int mt) {
-        const uint32_t t = uint32_t(mt) * uint32_t(nb) * 5120u;
+        const uint32_t t = uint32_t(mt) * uint32_t(nb) * 4096u;
 #pragma unroll
         for (int i = 0; i < 4; ++i) p.x.a[i] = ld128(rx, va + 4096u * blk + 1024u * i, t);
-        if constexpr (TY == kIQ1_M) p.x.a[4] = ld128(rx, va + 1024u * blk, t + 4096u * nb);
+        if constexpr (TY == kIQ1_M) p.x.a[4] = ld128(rs, va + 1024u * blk, t / 4);
         p.d = ld128(rp, 64u * blk + 16u * e4, uint32_t(mt) * uint32_t(nb) * 64u);
     };
     Raw w0[2], w1[2];   // IQ2
@@ -1199,12 +1203,13 @@ hipError_t launch_grouped(GroupArgs args, int gu_types, int dn_types, int cus, h
         return hipErrorNotSupported;
     const bool trace = args.tq8x || args.tq8h || args.th || args.tint, iq2 = gu_types == 1 && dn_types == 2;
     if (trace && !iq2) return hipErrorNotSupported;
+    if (((gu_types & 4) && !args.xs) || ((dn_types & 4) && !args.hs)) return hipErrorInvalidValue;
     const GroupPlan plan = group_plan(args, gu_types, dn_types, trace, cus);
     args.cap = plan.multi ? 64 : 16;
     const int P = args.T * args.k, nbx = args.dim / 256, nbh = args.ff / 256;
     const auto grouped = [&](auto kernel, int nw = 12) { hipLaunchKernelGGL(kernel, dim3(cus), dim3(nw * 64), 0, s, args); };
-    const auto rows = [&](auto kernel, const float* src, int n, int nb, int8_t* q, float* d, uint8_t* tr) {
-        hipLaunchKernelGGL(kernel, dim3((n * nb + 3) / 4), dim3(256), 0, s, src, n, nb, q, d, args.pos, args.k, args.err, tr);
+    const auto rows = [&](auto kernel, const float* src, int n, int nb, int8_t* q, int8_t* sums, float* d, uint8_t* tr) {
+        hipLaunchKernelGGL(kernel, dim3((n * nb + 3) / 4), dim3(256), 0, s, src, n, nb, q, sums, d, args.pos, args.k, args.err, tr);
     };
     // sums by eights (next_chain), where a row has more than eight blocks: without, it is
     // one chain all the same, and several-type kernels spill less (1024 x 512, 256 tokens
@@ -1216,13 +1221,13 @@ hipError_t launch_grouped(GroupArgs args, int gu_types, int dn_types, int cus, h
     args.dn_first = dn_types == 2 || dn_types == 4 ? cus : 0;
     hipLaunchKernelGGL(bucket_kernel, dim3(1), dim3(1024), 0, s, args);
     if (trace) {   // the parity trace (separate instances)
-        rows((q8k_rows_kernel<ROWS_X, false, true>), args.x, args.T, nbx, args.xq, args.xd, args.tq8x);
+        rows((q8k_rows_kernel<ROWS_X, false, true>), args.x, args.T, nbx, args.xq, args.xs, args.xd, args.tq8x);
         grouped(grouped_kernel<true, 1, NW, 1, true, false>);
-        rows((q8k_rows_kernel<ROWS_H, false, true>), args.h, P, nbh, args.hq, args.hd, args.tq8h);
+        rows((q8k_rows_kernel<ROWS_H, false, true>), args.h, P, nbh, args.hq, args.hs, args.hd, args.tq8h);
         grouped(grouped_kernel<false, 2, NW, 1, true, false>);
     } else {
         rows(gu_types & 4 ? q8k_rows_kernel<ROWS_X, true, false> : q8k_rows_kernel<ROWS_X, false, false>, args.x, args.T, nbx,
-             args.xq, args.xd, nullptr);
+             args.xq, args.xs, args.xd, nullptr);
         if (gu_types == 1) {
             if (plan.gu8) sums(gu_f8, grouped_kernel<true, 1, 8, 4, false, false>, grouped_kernel<true, 1, 8, 4, false, true>, 8);
             else sums(gu_f8, grouped_kernel<true, 1, NW, 1, false, false>, grouped_kernel<true, 1, NW, 1, false, true>, NW);
@@ -1234,7 +1239,7 @@ hipError_t launch_grouped(GroupArgs args, int gu_types, int dn_types, int cus, h
             else sums(gu_f8, grouped_kernel<true, 7, NWM, 1, false, false>, grouped_kernel<true, 7, NWM, 1, false, true>, NWM);
         }
         rows(dn_types & 4 ? q8k_rows_kernel<ROWS_H, true, false> : q8k_rows_kernel<ROWS_H, false, false>, args.h, P, nbh,
-             args.hq, args.hd, nullptr);
+             args.hq, args.hs, args.hd, nullptr);
         if (plan.dn_half) {   // IQ2 layers only
             grouped(grouped_kernel<false, 2, NW, 1, false, false, 1>);
         } else if (dn_types == 2) {

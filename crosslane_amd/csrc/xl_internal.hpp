@@ -131,7 +131,8 @@ struct GroupArgs {
     int T, k, n_experts, dim, ff;
     // Slots: tile i of 16 pairs owns slots 16 i .. 16 i + 15; a task is up to cap
     // pairs of one expert (cap a multiple of 16), in consecutive tiles.
-    int8_t* xq; float* xd;      // Q8_K(x): quants per tile (5/4 * 16 * dim bytes each, the MFMA order), scales per slot
+    int8_t* xq; float* xd;      // Q8_K(x): quants per tile (16 * dim bytes each, the MFMA order), scales per slot
+    int8_t* xs;                 // sums of 8 quants for IQ1_M gate/up (4 * dim bytes per tile), null without
     int32_t* order;             // pair of each used slot (16 * max tiles)
     int32_t* pos;               // slot of each pair (P; -1 for a bad id), with order bits (xl_grouped.hip)
     int4* tasks; int4* dtasks;  // (expert, first slot, pairs, 0) per task, by gate type and by down type
@@ -140,6 +141,7 @@ struct GroupArgs {
     int gu_first, dn_first;     // the queues' first bundles
     float* h;                   // P * ff
     int8_t* hq; float* hd;      // Q8_K(h): as xq and xd, of ff
+    int8_t* hs;                 // as xs, for IQ1_M down
     float* y;                   // P * dim
     const uint64_t* tables;     // expanded codebooks (kLayer3TableBytes)
     int* err;

@@ -63,10 +63,12 @@ typedef struct xl_config {
     int32_t max_picks;     /* top-k bound, 1..16 (reference kPicks = 8, model_meta.hpp:18) */
     int32_t max_tokens;    /* grouped-path token bound (0 = grouped path unused). Its
                               workspace, with P = max_tokens * max_picks: about
-                              20 * (P / 16 + min(P, n_experts) + 1) * (dim + ff) bytes
+                              16 * (P / 16 + min(P, n_experts) + 1) * (dim + ff) bytes
                               of per-slot quants plus 4 * P * (dim + ff) bytes of h
-                              and per-pick rows (~200 MB at 512 tokens, 8 picks,
-                              384 experts, 4096 x 3072) */
+                              and per-pick rows (~190 MB at 512 tokens, 8 picks,
+                              384 experts, 4096 x 3072). xl_bank_create adds a
+                              quarter of the quants' dim part where a gate or up
+                              matrix is IQ1_M, of their ff part where a down is */
     float swiglu_limit;    /* SwiGLU limit (model_meta.hpp:34 `lim`, the pack's swiglu_limit):
                               > 0 clamps g to <= lim and u to [-lim, lim] before
                               SiLU(g) * u (q8k_core.hpp:92-95); <= 0: no clamp */
@@ -75,7 +77,7 @@ typedef struct xl_config {
 typedef struct xl_bank_info {
     uint64_t payload_bytes;    /* ggml bytes of every resident matrix */
     uint64_t allocated_bytes;  /* device bytes held by the bank (256-B aligned planes) */
-    uint64_t workspace_bytes;  /* device bytes of the per-call workspace */
+    uint64_t workspace_bytes;  /* device bytes of the per-call workspace (with xl_bank_create's part) */
     int32_t n_layers, n_experts;
     int32_t generated;         /* 1 after xl_bank_generate */
     int32_t reserved;

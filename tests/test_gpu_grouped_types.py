@@ -148,3 +148,17 @@ def test_plans_keep_the_bits(dim, ff, E, T, k):
     assert int((out.view(torch.int32) != traced.view(torch.int32)).sum()) == 0
     assert T == 1 or int((out[T // 2] != shared[T // 2]).sum()) == 0
     assert float(out.abs().max()) > 0
+
+
+@pytest.mark.parametrize("gu,dn", [(16, 17), (29, 17), (16, 29), (29, 29)])
+def test_only_iq1_banks_have_its_workspace(gu, dn):
+    """The sums that IQ1_M's MFMAs take are allocated with a bank that has IQ1_M
+    matrices of that role, and with no other."""
+    dim, ff, E, T, k = 1024, 512, 8, 64, 4
+    types = np.zeros((1, E, 3), np.int32)
+    types[..., :2], types[..., 2] = gu, dn
+    tiles = T * k // 16 + E + 1
+    with xl.Lane(dim, ff, 1, E, np.full((1, E, 3), 16, np.int32), max_picks=k, max_tokens=T) as lane:
+        least = lane.info()["workspace_bytes"]
+    with xl.Lane(dim, ff, 1, E, types, max_picks=k, max_tokens=T) as lane:
+        assert lane.info()["workspace_bytes"] - least == 4 * tiles * (dim * (gu == 29) + ff * (dn == 29))
