@@ -41,17 +41,17 @@
 // filling its LDS tables for that type.
 //
 // Weights stream from HBM through registers: each wave loads its rows' next block
-// while it computes the current one, and touches the line four blocks ahead with
-// one dword per row so that it is in L2 when the real loads come. The texture data
-// path costs one cycle per cache access, and a quad of lanes makes one access only
-// when it reads 64 contiguous bytes: so each lane loads just the 16 B of its row's
-// block that it decodes (the entries then move between lane groups by permlane
-// swaps), activations are laid out so that a quad's four slots are adjacent, and
-// the small per-block scales are staged once per tile in the wave's own LDS. An
-// IQ1_M lane needs 8, 4 and 8 bytes of three planes per block: loaded directly,
-// those kept the texture unit busy for the whole kernel (1,415 us for gate/up of
-// 512 tokens at 4096 x 3072, 384 experts), so four blocks of the 16 rows come as
-// whole 16-byte pieces and go through the wave's LDS.
+// while it computes the current one (one dword per row that touched the line four
+// blocks ahead made calls up to 22 % slower: 13 tokens, 384 experts; the other waves
+// cover the latency). The texture data path costs one cycle per cache access, and a
+// quad of lanes makes one access only when it reads 64 contiguous bytes: so each lane
+// loads just the 16 B of its row's block that it decodes (the entries then move
+// between lane groups by permlane swaps), activations are laid out so that a quad's
+// four slots are adjacent, and the small per-block scales are staged once per tile in
+// the wave's own LDS. An IQ1_M lane needs 8, 4 and 8 bytes of three planes per block:
+// loaded directly, those kept the texture unit busy for the whole kernel (1,415 us for
+// gate/up of 512 tokens at 4096 x 3072, 384 experts), so four blocks of the 16 rows
+// come as whole 16-byte pieces and go through the wave's LDS.
 //
 // Bound by the decode work per weight byte: at 512 tokens (4096 x 3072, 384 experts,
 // 6 picks) the IQ2 gate/up launch issues VALU on 71 % of its cycles, LDS lookups fill
@@ -377,9 +377,6 @@ __global__ __launch_bounds__(256) void q8k_rows_kernel(const float* __restrict__
     }
 }
 
-// Keeps a value alive without storing it (the L2 line touches).
-__device__ __forceinline__ void sink(uint32_t& acc, uint32_t v) { acc ^= v; }
-
 // Buffer loads: the base in a scalar descriptor, the per-lane byte offset in
 // voffset, a uniform plane offset in soffset.
 typedef uint32_t v4u32 __attribute__((ext_vector_type(4)));
@@ -486,8 +483,6 @@ __device__ __forceinline__ void load_raw(Raw& o, const Stream& st, int blk, int 
     o.q = ld128(st.r, 64u * b + 16u * e4);
     if constexpr (TY == kIQ2_XS) o.s = ld64(st.r, 8u * b, st.o1);
 }
-// Touches the line of block blk (a row's blocks share a line by twos).
-__device__ __forceinline__ uint32_t touch(const Stream& st, int blk) { return ld32(st.r, 64u * (st.at + uint32_t(blk))); }
 // Four IQ1_M blocks (blk0 .. + 3, past the row's end the last one) of a stream's 16
 // rows, as pieces: row0nb = the stream's first row * nb.
 struct Raw1 {
@@ -672,8 +667,7 @@ __device__ __forceinline__ void next_chain(float* acc, float* total, int b, int 
 }
 // TR: also write each pair's block integers (GroupArgs::tint).
 template <bool GU, int TY, bool TR, bool DB, bool F8, int NS>
-__device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int tl, uint8_t* lds, uint8_t* wl, int lane,
-                                        uint32_t& sunk) {
+__device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int tl, uint8_t* lds, uint8_t* wl, int lane) {
     const int col = lane & 15, e4 = lane >> 4, nb = (GU ? a.dim : a.ff) / 256;
     const uint32_t mk = e4 < 2 ? ~0u : 0u;   // lanes of entries 0, 1
     static_assert(!GU || NS == 2, "gate and up");
@@ -700,13 +694,11 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
         if constexpr (TY == kIQ1_M) x.a[4] = ld128(rs, va + 1024u * blk);
     };
     Raw w0[NS], w1[NS];   // IQ2
-    uint32_t t0 = 0, t2 = 0;
     auto load = [&](Raw (&w)[NS], Act<TY>& x, int blk) {
 #pragma unroll
         for (int s = 0; s < NS; ++s) load_raw<TY>(w[s], st[s], blk, e4);
         load_x(x, blk);
     };
-    auto touch2 = [&](int blk) { return touch(st[0], blk) ^ touch(st[NS - 1], blk); };
     Raw1 r1[NS];         // IQ1_M
     if constexpr (TY == kIQ1_M) {
 #pragma unroll
@@ -714,8 +706,6 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
         if (DB) load_x(x0, 0);
     } else {
         load(w0, x0, 0);
-        t0 = touch2(min(1, nb - 1));
-        t2 = touch2(min(3, nb - 1));
     }
     // the tile's pair scales and rows' scales into the wave's own LDS
     float* pd = reinterpret_cast<float*>(wl);
@@ -803,28 +793,22 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
             }
         } else {
             // Two operand sets alternate over a 4-step unrolled loop (no register copies,
-            // so no wait ever covers a load issued in the same step); line touches four
-            // blocks ahead in fixed registers, one per line of two blocks.
+            // so no wait ever covers a load issued in the same step).
             for (int b = 0; b < nb; b += 4) {
                 if (b > 0) next_chain<F8, 4 * NS>(acc[0], total[0], b, nb);
                 load(w1, x1, min(b + 1, nb - 1));
-                sink(sunk, t0);
-                t0 = touch2(min(b + 5, nb - 1));
                 __builtin_amdgcn_sched_barrier(0);   // the loads stay ahead of the compute
                 compute(w0, x0);
                 load(w0, x0, min(b + 2, nb - 1));
                 __builtin_amdgcn_sched_barrier(0);
                 if (b + 1 < nb) compute(w1, x1);
                 load(w1, x1, min(b + 3, nb - 1));
-                sink(sunk, t2);
-                t2 = touch2(min(b + 7, nb - 1));
                 __builtin_amdgcn_sched_barrier(0);
                 if (b + 2 < nb) compute(w0, x0);
                 load(w0, x0, min(b + 4, nb - 1));
                 __builtin_amdgcn_sched_barrier(0);
                 if (b + 3 < nb) compute(w1, x1);
             }
-            sink(sunk, t0 ^ t2);
         }
         next_chain<F8, 4 * NS>(acc[0], total[0], 0, nb);
 #pragma unroll
@@ -849,8 +833,7 @@ __device__ __forceinline__ void do_tile(const GroupArgs& a, const int4& tk, int 
 // operations per pair); the pair scales come from memory (LDS has no room for NT
 // sets beside the tables), one step ahead with the activations.
 template <bool GU, int TY, int NT, bool F8>
-__device__ __forceinline__ void do_tiles(const GroupArgs& a, const int4& tk, int tl, uint8_t* lds, uint8_t* wl, int lane,
-                                         uint32_t& sunk) {
+__device__ __forceinline__ void do_tiles(const GroupArgs& a, const int4& tk, int tl, uint8_t* lds, uint8_t* wl, int lane) {
     const int col = lane & 15, e4 = lane >> 4, nb = (GU ? a.dim : a.ff) / 256;
     const uint32_t mk = e4 < 2 ? ~0u : 0u;
     Stream st[2];
@@ -881,19 +864,16 @@ __device__ __forceinline__ void do_tiles(const GroupArgs& a, const int4& tk, int
         p.d = ld128(rp, 64u * blk + 16u * e4, uint32_t(mt) * uint32_t(nb) * 64u);
     };
     Raw w0[2], w1[2];   // IQ2
-    uint32_t t0 = 0;
     auto load_w = [&](Raw (&w)[2], int blk) {
 #pragma unroll
         for (int s = 0; s < 2; ++s) load_raw<TY>(w[s], st[s], blk, e4);
     };
-    auto touch2 = [&](int blk) { return touch(st[0], blk) ^ touch(st[1], blk); };
     Raw1 r1[2];         // IQ1_M
     if constexpr (TY == kIQ1_M) {
 #pragma unroll
         for (int s = 0; s < 2; ++s) load_raw1(r1[s], st[s], row0nb[s], 0, nb, lane);
     } else {
         load_w(w0, 0);
-        t0 = touch2(min(3, nb - 1));
     }
     load_p(p0, 0, 0);
     uint16_t* rd = reinterpret_cast<uint16_t*>(wl + 64 * kGrpNb);
@@ -963,13 +943,10 @@ __device__ __forceinline__ void do_tiles(const GroupArgs& a, const int4& tk, int
         for (int b = 0; b < nb; b += 2) {
             if (b > 0) next_chain<F8, 8 * NT>(acc[0][0], total[0][0], b, nb);
             load_w(w1, min(b + 1, nb - 1));
-            sink(sunk, t0);
-            t0 = touch2(min(b + 5, nb - 1));
             block(w0, b, even);
             load_w(w0, min(b + 2, nb - 1));
             if (b + 1 < nb) block(w1, b + 1, second);
         }
-        sink(sunk, t0);
     }
     next_chain<F8, 8 * NT>(acc[0][0], total[0][0], 0, nb);
 #pragma unroll
@@ -1012,7 +989,6 @@ __global__ __launch_bounds__(NW * 64, 1) void grouped_kernel(GroupArgs a) {
         const int64_t at = int64_t(all) * (2 * blockIdx.x + 1);
         first = at < int64_t(c0) * 2 * gridDim.x ? 0 : at < int64_t(c1) * 2 * gridDim.x ? 1 : 2;
     }
-    uint32_t sunk = 0;
     for (int i = 0; i < (MASK == 7 ? 3 : 1); ++i) {
         const int ti = MASK == 7 ? (first + i) % 3 : MASK == 1 ? 0 : MASK == 2 ? 1 : 2;
         const int base = ti == 0 ? 0 : ti == 1 ? n[0] : n[0] + n[1];   // the type's tasks in the list
@@ -1035,24 +1011,9 @@ __global__ __launch_bounds__(NW * 64, 1) void grouped_kernel(GroupArgs a) {
             __syncthreads();
         }
         if (!s_open) continue;   // nothing left of this type (workgroup-uniform)
-        uint32_t warm[2] = {0, 0};
-        if (MASK != 7) {   // the chain of loads to the wave's first rows, under the tables' fill
-            const int ft = even ? start + wv : int(blockIdx.x) * bs + wv;
-            if (bs == 0) break;
-            if (wv < bs && ft < total) {
-                const int task = ft / tiles, tl = ft - task * tiles, nb = (GU ? a.dim : a.ff) / 256;
-                const int4 tk = task_at((GU ? a.tasks : a.dtasks) + base, task);
-#pragma unroll
-                for (int s = 0; s < NS; ++s) {
-                    const MatRef m = mat_at(a.descs, tk.x, GU ? s : 2);
-                    const int row = (GU ? 16 * tl : 16 * (NS * tl + s)) + (lane & 15);
-                    warm[s] = ld32(rsrc(m.base), (ti == 2 ? 32u : 64u) * uint32_t(row * nb));
-                }
-            }
-        }
+        if (MASK != 7 && bs == 0) break;   // workgroup-uniform
         fill_tables<NW * 64>(lds, ti == 0 ? kIQ2_XXS : ti == 1 ? kIQ2_XS : kIQ1_M, a.tables, t);
         __syncthreads();
-        sink(sunk, warm[0] ^ warm[1]);
         for (;;) {
             uint32_t got = 0;
             for (;;) {   // this wave's next tile
@@ -1082,12 +1043,12 @@ __global__ __launch_bounds__(NW * 64, 1) void grouped_kernel(GroupArgs a) {
             const int4 tk = task_at((GU ? a.tasks : a.dtasks) + base, task);
             const auto tile_of = [&]<int TY>() {
                 if constexpr (MT == 1) {
-                    do_tile<GU, TY, TR, NW <= 8, F8, NS>(a, tk, tl, lds, wl, lane, sunk);
+                    do_tile<GU, TY, TR, NW <= 8, F8, NS>(a, tk, tl, lds, wl, lane);
                 } else {
-                    if (tk.z <= 16) do_tiles<GU, TY, 1, F8>(a, tk, tl, lds, wl, lane, sunk);
-                    else if (tk.z <= 32) do_tiles<GU, TY, 2, F8>(a, tk, tl, lds, wl, lane, sunk);
-                    else if (tk.z <= 48) do_tiles<GU, TY, 3, F8>(a, tk, tl, lds, wl, lane, sunk);
-                    else do_tiles<GU, TY, 4, F8>(a, tk, tl, lds, wl, lane, sunk);
+                    if (tk.z <= 16) do_tiles<GU, TY, 1, F8>(a, tk, tl, lds, wl, lane);
+                    else if (tk.z <= 32) do_tiles<GU, TY, 2, F8>(a, tk, tl, lds, wl, lane);
+                    else if (tk.z <= 48) do_tiles<GU, TY, 3, F8>(a, tk, tl, lds, wl, lane);
+                    else do_tiles<GU, TY, 4, F8>(a, tk, tl, lds, wl, lane);
                 }
             };
             if (MASK == 1 || (MASK == 7 && ti == 0)) tile_of.template operator()<kIQ2_XXS>();
@@ -1095,7 +1056,6 @@ __global__ __launch_bounds__(NW * 64, 1) void grouped_kernel(GroupArgs a) {
             else tile_of.template operator()<kIQ1_M>();
         }
     }
-    if (sunk == 0x9e3779b9u && lane == 64) (GU ? a.h : a.y)[0] = 0.0f;   // never true (lane < 64): keeps the touches
 }
 
 // ---------------------------------------------------------------------------
