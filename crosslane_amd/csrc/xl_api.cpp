@@ -174,7 +174,8 @@ struct xl_context {
     int path = 1;
     // Grouped path: 1 = the MFMA kernels where the layer's types allow, else one
     // layer call per token (default); 0 = per-token calls only; 2 = the MFMA
-    // kernels only (a layer they cannot run is an error). XL_GROUPED_PATH selects.
+    // kernels only, and of those only the IQ2_XXS gate/up + IQ2_XS down ones (another
+    // layer is an error). XL_GROUPED_PATH selects.
     int gpath = 1;
     float* hbuf = nullptr;      // streaming kernel's h exchange (2 x kHBufWords, sentinel-filled)
     // grouped path (xl_grouped.hip), sized by max_tokens * max_picks pairs
@@ -1127,9 +1128,9 @@ int32_t xl_expert_forward(xl_context* ctx, int32_t layer, int32_t expert, const 
 
 namespace {
 
-// Enqueues T tokens of layer `layer` on stream s: the grouped MFMA kernels when
-// the layer's gate/up are IQ2_XXS and its down IQ2_XS, otherwise one layer
-// call per token. All pointers are device pointers.
+// Enqueues T tokens of layer `layer` on stream s: the grouped MFMA kernels (layers
+// of other types than IQ2_XXS gate/up with IQ2_XS down from kGroupAnyTokens tokens
+// on), otherwise one layer call per token. All pointers are device pointers.
 void enqueue_grouped(xl_context* ctx, int32_t layer, int32_t T, int32_t k, const int32_t* d_ids, const float* d_w,
                      const float* d_x, const float* d_shared, float* d_out, hipStream_t s, LayerTrace* tr = nullptr) {
     const int dim = ctx->cfg.dim, E = ctx->cfg.n_experts;
@@ -1165,8 +1166,8 @@ void enqueue_grouped(xl_context* ctx, int32_t layer, int32_t T, int32_t k, const
         if (e != hipErrorNotSupported) hip_check(e, "grouped launch");
         (void)hipGetLastError();
     }
-    need(ctx->gpath != 2, XL_E_ARG, "XL_GROUPED_PATH=2: the grouped MFMA kernels cannot run this layer");
-    need(tr == nullptr, XL_E_ARG, "trace: this layer does not run on the grouped MFMA kernels");
+    need(ctx->gpath != 2, XL_E_ARG, "XL_GROUPED_PATH=2 admits only layers of IQ2_XXS gate/up and IQ2_XS down with ff <= 4096 and at most 8192 experts");
+    need(tr == nullptr, XL_E_ARG, "trace: only layers of IQ2_XXS gate/up and IQ2_XS down, within the grouped MFMA kernels' limits");
     for (int t = 0; t < T; ++t)
         enqueue_layer(ctx, layer, d_ids + size_t(t) * k, d_w + size_t(t) * k, k, d_x + size_t(t) * dim,
                       d_shared ? d_shared + size_t(t) * dim : nullptr, d_out + size_t(t) * dim, s);

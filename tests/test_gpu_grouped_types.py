@@ -54,10 +54,8 @@ def test_grouped_types(orc, kind, dim, ff, E, T, k, skew, lim):
         assert lane.launch_counts() == counts          # no per-token layer call served it
         assert np.array_equal(got.view(np.uint32), lane.grouped_forward(0, ids, w, x, shared).view(np.uint32))
         per = np.stack([lane.layer_forward(0, ids[t], w[t], x[t], shared[t]) for t in range(T)])
-    # a quant of h that rounds the other way moves a token past the bar on ~0.1 % of the tokens
-    far = [t for t in range(T) if max_rel(got[t], per[t]) > TOL]
-    assert len(far) <= 1 + T // 100 and max_rel(got, per) < 5 * TOL, (far, max_rel(got, per))
-    for t in sorted({0, T // 2, T - 1} - set(far)):
+    assert max(max_rel(got[t], per[t]) for t in range(T)) < TOL
+    for t in sorted({0, T // 2, T - 1}):
         rows = []
         for e in ids[t]:
             tt = tuple(int(v) for v in types[0, e])
@@ -91,6 +89,38 @@ def test_tasks_of_several_tiles(dim, ff):
         lane.sync()
     assert float(out.abs().max()) > 0
     assert torch.equal(out.view(torch.int32), traced.view(torch.int32))
+
+
+@pytest.mark.parametrize("dim,ff", [(768, 1024), (2304, 1024), (1024, 3072), (4096, 2304)])
+@pytest.mark.parametrize("kind", ["iq1", "mixed", "swapped", "split"])
+def test_tasks_of_several_tiles_of_any_types(kind, dim, ff):
+    """The same pairs in one call, about 43 per expert (tasks of 1 to 4 tiles and their
+    remainders), and in calls of 512 pairs or fewer, 8 per expert (16-pair tasks,
+    other kernels): the same bits. Rows of an odd number of blocks, and of more than
+    eight (whose float sums are chains of eight)."""
+    counts = [16, 17, 32, 33, 48, 49, 64, 65, 1, 129, 15, 50, 63]
+    print(f"[gpu-step] tasks of several tiles {kind} {dim}x{ff}", flush=True)
+    E = 64
+    per = np.resize(counts, E)
+    T = int(per.sum())
+    rng = np.random.default_rng(dim + ff)
+    ids = rng.permutation(np.repeat(np.arange(E), per)).astype(np.int32).reshape(T, 1)
+    types = type_map(kind, E, rng)
+    d_ids, d_w, d_x = (torch.from_numpy(a).cuda() for a in (ids, rng.random((T, 1)).astype(np.float32),
+                                                            rng.standard_normal((T, dim)).astype(np.float32)))
+    out, parts = torch.zeros((T, dim), device="cuda"), torch.zeros((T, dim), device="cuda")
+    torch.cuda.synchronize()
+    with xl.Lane(dim, ff, 1, E, types, max_picks=1, max_tokens=T) as lane:
+        lane.generate(seed=4)
+        lane.grouped_forward_async(0, d_ids, d_w, d_x, out)
+        for t in range(0, T, 512):
+            n = min(512, T - t) if T - t >= 600 else T - t   # no call below the 13 tokens of the grouped kernels
+            lane.grouped_forward_async(0, d_ids[t:t + n], d_w[t:t + n], d_x[t:t + n], parts[t:t + n])
+            if t + n == T:
+                break
+        lane.sync()
+    assert float(out.abs().max()) > 0
+    assert int((out.view(torch.int32) != parts.view(torch.int32)).sum()) == 0
 
 
 @pytest.mark.parametrize("dim,ff", [(4096, 3072), (5120, 2304), (1024, 512)])
