@@ -54,9 +54,10 @@
 // come as whole 16-byte pieces and go through the wave's LDS.
 //
 // Bound by the decode work per weight byte: at 512 tokens (4096 x 3072, 384 experts,
-// 6 picks) the IQ2 gate/up launch issues VALU on 71 % of its cycles, LDS lookups fill
-// 38 %. Whole calls there: IQ2 1,422 us (1,463 with workgroup barriers per item),
-// IQ1_M 1,265, mixed types 1,426 (10,999 and 12,992 as 512 layer calls).
+// 6 picks, IQ2) VALU issue takes 79 % of the gate/up launch's SIMD cycles (765 us) and
+// 71 % of the down launch's (531), LDS 36 % of its cycles in both; at 2,048 tokens, by
+// 64 pairs, 82 and 84 %. Whole calls at 512 tokens: IQ2 1,307 to 1,350 us, IQ1_M 1,149,
+// mixed types 1,335 (10,999 and 12,992 as 512 layer calls).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1155,11 +1156,12 @@ GroupPlan group_plan(const GroupArgs& a, int gu_types, int dn_types, bool trace,
 }  // namespace
 
 hipError_t launch_grouped(GroupArgs args, int gu_types, int dn_types, int cus, hipStream_t s) {
-    // waves per workgroup: 3 per SIMD; layers of several types 2, whose kernel spills
-    // 50 registers at 3 (512 tokens, 4096 x 3072, 384 experts: 1,426 against 1,494 us)
+    // Waves per workgroup: 3 per SIMD; layers of several types 2: at 3 their kernels spill
+    // 39 to 60 registers (512 tokens, 4096 x 3072, 384 experts: 1,512 us against 1,335), at
+    // 2 up to 16, and 44 to 90 with 64-pair tasks, which still win (kMultiPairsMix).
     constexpr int NW = 12, NWM = 8;
     if (args.T < 1 || args.k < 1 || args.k > 16 || args.n_experts > kGroupMaxExperts || args.dim % 256 || args.ff % 256 ||
-        args.dim > kGrpNb * 256 || args.ff > 4096)
+        args.dim > kGrpNb * 256 || args.ff > 4096)   // (longer hidden rows would fit: not measured)
         return hipErrorNotSupported;
     const bool trace = args.tq8x || args.tq8h || args.th || args.tint, iq2 = gu_types == 1 && dn_types == 2;
     if (trace && !iq2) return hipErrorNotSupported;

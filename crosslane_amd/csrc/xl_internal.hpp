@@ -156,14 +156,16 @@ struct GroupArgs {
     int32_t* tint;
 };
 // Tokens from which layers that are not IQ2_XXS gate/up + IQ2_XS down run grouped.
-// Measured at 4096 x 3072, 384 experts, 6 picks: 13 tokens 327 us (mixed types) and
-// 265 us (IQ1_M) grouped against 354 and 298 us by layer calls, about level at 12
-// (fewer experts or smaller shapes gain earlier: 13 tokens at 1024 x 512 take 41 us
-// against 158). Below it a call keeps the bits of its tokens' single layer calls; from it
-// on the float sums have another order, no further from 64 bits (next_chain).
+// The line lies where no call loses: of 13, 16 and 24 tokens at five shapes, 64 and 384
+// experts and 1 to 16 picks the closest is 4096 x 3072, 384 experts, 6 picks, mixed types
+// (13 tokens 320 us grouped against 336 by layer calls; IQ1_M 252 against 282), about
+// level at 12. Smaller shapes, fewer experts or picks would gain with fewer tokens (13 at
+// 1024 x 512 take 41 us against 158); that is not used yet. Below the line a call keeps the
+// bits of its tokens' single layer calls; from it on the float sums have another order,
+// no further from 64 bits (next_chain).
 constexpr int kGroupAnyTokens = 13;
-constexpr int kGroupMaxExperts = 8192;
-constexpr int kRouteMaxExperts = 4096;   // router: scores and keys of one token in LDS   // experts per layer the bucket kernel counts in LDS
+constexpr int kGroupMaxExperts = 8192;   // experts per layer the bucket kernel counts in LDS
+constexpr int kRouteMaxExperts = 4096;   // router: scores and keys of one token in LDS
 // Tiles (and at most as many tasks) for P pairs: one per started 16 pairs of an expert.
 inline int64_t group_max_tiles(int64_t P, int64_t n_experts) { return P / 16 + (P < n_experts ? P : n_experts) + 1; }
 constexpr int kLayer3TableBytes = 24576;   // expanded codebooks of the single-launch kernel

@@ -25,12 +25,15 @@
 // waves' chains through LDS (c and c ^ 2, then c and c ^ 1), the next two a wave's
 // own four, the last the two parities.
 //
-// What bounds it: the float part, five VALU instructions per output and
-// sub-block for Q4_K / Q5_K and Q6_K (three for Q8_0) against a quarter of an
-// MFMA; decode and scales add a third at 32 tokens (VALU issue ~90 % of the
-// gate/up launch). 512 tokens, 4096 x 3072, Q5_K gate/up and Q6_K down: 242 us,
-// 160 TFLOP/s (132 us gate/up, 96 us down; the row kernels, which decode every
-// weight once per token: 2,913 us); 16 tokens: 35 us (120).
+// What bounds it: VALU issue, and the copies to LDS, whose latency is not hidden
+// (stage_step). The float part is five VALU instructions per output and sub-block for
+// Q4_K / Q5_K and Q6_K (three for Q8_0) against a quarter of an MFMA: at 512 tokens of
+// 4096 x 3072 77 of the 160 us that all VALU instructions take to issue; the rest is
+// decode, scales and the sums' exchange. There, Q5_K gate/up and Q6_K down: 205 us, 189
+// TFLOP/s (traced 127 us gate/up, VALU issue 84 % of its SIMD cycles, 95 us down, 65 %; the
+// row kernels, which decode every weight once per token: 2,913 us); 16 tokens: 32 us
+// (120). The 32-token instances spill (Q8_0 13, Q4_K 2, Q5_K 9, Q6_K 41 registers of
+// gate/up; Q5_K 2, Q6_K 18 of down).
 #include <hip/hip_runtime.h>
 
 #include "xl_dev.hpp"
@@ -80,9 +83,11 @@ __device__ __forceinline__ ActTile act_tile(const int8_t* q, const float* d, int
 __host__ __device__ constexpr int row_block_bytes(int ty) { return ty == kQ8_0 ? 8 * 34 : dense_block_bytes(ty); }
 
 // The weights go through LDS, 32 rows of four 256-value blocks at a time (one per
-// c), copied there directly as whole 16-byte pieces one step ahead (a lane's
-// 8-byte slices straight from memory cost the texture unit one access per lane,
-// and bounded the kernel). Row stride: an odd number of pieces, so that the 16
+// c), copied there directly as whole 16-byte pieces (a lane's 8-byte slices straight
+// from memory cost the texture unit one access per lane, and bounded the kernel). The
+// copies of step s + 1 go out before the products of step s, but not ahead of its first
+// LDS read: the compiler cannot tell the halves of the stage apart and waits there for
+// every copy in flight, so that each step shows a copy's latency. Row stride: an odd number of pieces, so that the 16
 // rows' slices fall into different banks. A Q6_K block starts at any even byte:
 // its pieces start at the 16-byte boundary before it and 14 hold it (n and k are
 // multiples of 256, so that the last block's pieces end with the matrix).
