@@ -384,7 +384,8 @@ hipError_t launch_gate_up32(const ExpertDesc* descs, const int32_t* ids, int pic
 }
 
 // hipErrorNotSupported: the hidden rows of all picks or a workgroup's outputs do
-// not fit beside the 128 KB of tables (more than 8 picks of 3,072 values);
+// not fit beside the 128 KB of tables (more than 8 picks of 3,072 values; one
+// limit for all instances, though IQ1_M's tables of 32 KB would leave room);
 // mv32_kernel, which stages neither, takes those.
 hipError_t launch_down32(const ExpertDesc* descs, const int32_t* ids, int picks, int n_experts, int mask, int n, int k,
                          const int8_t* q, const float* d, float* y, const Mv32Comb& cb, const uint64_t* tables, int cus,
